@@ -30,6 +30,13 @@ __device__ __forceinline__ float f16_bits_to_f32(uint32_t bits) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)bits);
 }
 
+// i % m; a 64-bit remainder is some 50 instructions, so it is taken only where
+// i needs it (12288x4096 with a column scale, us: GF4 44.9 -> 42.3, Q4_K 64.0
+// -> 60.3, GF2 52.8 -> 47.3).
+__device__ __forceinline__ uint32_t mod_u64(uint64_t i, uint32_t m) {
+    return (i >> 32) == 0 ? (uint32_t)i % m : (uint32_t)(i % m);
+}
+
 // Grid-stride loops keep the grid at a fixed size for any tensor.
 constexpr int kEncodeThreads = 256;
 constexpr int kEncodeBlocks = 2048;
@@ -45,7 +52,7 @@ __global__ __launch_bounds__(kEncodeThreads) void gf4_pack_kernel(const float* _
         const float4_t hi = *reinterpret_cast<const float4_t*>(src + 8 * i + 4);
         float v[8] = {lo.x, lo.y, lo.z, lo.w, hi.x, hi.y, hi.z, hi.w};
         if (col_scale) {
-            const uint32_t c0 = 8u * (uint32_t)(i % words_per_row);
+            const uint32_t c0 = 8u * mod_u64(i, words_per_row);
             const float4_t s0 = *reinterpret_cast<const float4_t*>(col_scale + c0);
             const float4_t s1 = *reinterpret_cast<const float4_t*>(col_scale + c0 + 4);
             const float s[8] = {s0.x, s0.y, s0.z, s0.w, s1.x, s1.y, s1.z, s1.w};
@@ -79,48 +86,117 @@ __global__ __launch_bounds__(kEncodeThreads) void gf4_pack_kernel(const float* _
     }
 }
 
-// One thread per q8_0 block: d = max|x| / 127, q = round_half_away(x * (1/d)).
-// One thread per GF2 super-block (256 columns = 16 groups of 16; this library's
-// encoder, the statement of oracle gf2_quantize):
+// Super-block encoders (GF2, Q4_K, Q5_K, Q6_K): one wave per 256-column
+// super-block, four consecutive columns per lane, so a super-block is one
+// coalesced 1 KB load, its group maxima are lane reductions and its packed
+// words one or two narrow stores; kSuperUnroll super-blocks' loads are in
+// flight per wave.  The encoders are bound by their fp32 reads and the IEEE
+// divides.  A thread per super-block (1 KB apart, three passes over its
+// columns) took 1061 us for Q4_K 12288x4096 with a column scale (0.22 TB/s);
+// this form takes 61 (3.8 TB/s; GF2 47, Q6_K 61).
+constexpr int kSuperUnroll = 4;
+constexpr int kEncodeWaves = kEncodeThreads / 64;
+
+// The lane's four columns of super-blocks i0 .. i0 + kSuperUnroll - 1
+// (clamped to the last one), times the column scale.
+__device__ __forceinline__ void load_super(const float* __restrict__ src, const float* __restrict__ col_scale,
+                                           uint64_t i0, uint64_t n_blocks, uint32_t blocks_per_row, int lane,
+                                           float (&v)[kSuperUnroll][4]) {
+    float4_t x[kSuperUnroll], s[kSuperUnroll];
+#pragma unroll
+    for (int u = 0; u < kSuperUnroll; ++u) {
+        const uint64_t i = i0 + u < n_blocks ? i0 + u : n_blocks - 1;
+        x[u] = *reinterpret_cast<const float4_t*>(src + 256 * i + 4 * lane);
+        if (col_scale)
+            s[u] = *reinterpret_cast<const float4_t*>(col_scale + 256u * mod_u64(i, blocks_per_row) + 4 * lane);
+    }
+#pragma unroll
+    for (int u = 0; u < kSuperUnroll; ++u)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) v[u][q] = col_scale ? __fmul_rn(x[u][q], s[u][q]) : x[u][q];
+}
+
+template <int CTRL>
+__device__ __forceinline__ float dpp_fmax(float v) {
+    return fmaxf(v, dpp_f32<CTRL>(v));
+}
+template <int CTRL>
+__device__ __forceinline__ float dpp_fmin(float v) {
+    return fminf(v, dpp_f32<CTRL>(v));
+}
+
+// r[q] = rint(fl(n[q] / d) * mul + add) in the IEEE steps that the formats
+// state, without an IEEE divide where it cannot matter: t = n * rcp(d) is
+// within a few ulp of the quotient, so for |t| < 256 both round to the same
+// integer unless t lies within 0.001 of a tie; only a wave that holds such a
+// lane (or a divisor outside rcp's accurate range) divides.  d != 0.
+// (Q4_K 12288x4096 with a column scale: 87.5 -> 64.0 us with this and the
+// shared sub-block arithmetic of k_quantize_kernel.)
+template <bool AFFINE>
+__device__ __forceinline__ void rint_div4(const float (&n)[4], float d, float (&r)[4]) {
+    const float inv = __builtin_amdgcn_rcpf(d);
+    float far = 0.0f, big = 0.0f;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+        float t = n[q] * inv;
+        if (AFFINE) t = __builtin_fmaf(t, 1.5f, 1.5f);
+        r[q] = rintf(t);
+        far = fmaxf(far, fabsf(t - r[q]));
+        big = fmaxf(big, fabsf(t));
+    }
+    const bool sure = far < 0.499f && big < 256.0f && fabsf(d) > 0x1p-100f && fabsf(d) < 0x1p+100f;
+    if (__any(!sure)) {
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const float t = __fdiv_rn(n[q], d);
+            r[q] = rintf(AFFINE ? __fadd_rn(__fmul_rn(t, 1.5f), 1.5f) : t);
+        }
+    }
+}
+
+// GF2 super-blocks (256 columns = 16 groups of 16; this library's encoder, the
+// statement of oracle gf2_quantize):
 //   b = e5m2(max |x|) (fp16 RNE, low byte rounded half-up), s = fp16(b << 8)
 //   t = x / s (0 where s == 0), q = clip(rint(t * 1.5 + 1.5), 0, 3)
 // written as the reference's super-block: 16 code words (code i of word w in
 // bits 2i, 2i+1 for column 16w + i) then the 16 scale bytes
-// (qw35-server/src/metal/qw35_gf2.metal:1-17).
+// (qw35-server/src/metal/qw35_gf2.metal:1-17).  A group is one quad of lanes.
 __global__ __launch_bounds__(kEncodeThreads) void gf2_pack_kernel(const float* __restrict__ src,
                                                                   const float* __restrict__ col_scale,
                                                                   uint8_t* __restrict__ dst, uint64_t n_blocks,
                                                                   uint32_t blocks_per_row) {
-    for (uint64_t i = (uint64_t)blockIdx.x * kEncodeThreads + threadIdx.x; i < n_blocks;
-         i += (uint64_t)gridDim.x * kEncodeThreads) {
-        const float* x = src + 256 * i;
-        const float* cs = col_scale ? col_scale + 256u * (uint32_t)(i % blocks_per_row) : nullptr;
-        uint32_t words[16];
-        uint32_t sb[4] = {0, 0, 0, 0};
-        for (int w = 0; w < 16; ++w) {
-            float v[16];
-            float amax = 0.0f;
-            for (int l = 0; l < 16; ++l) {
-                v[l] = cs ? __fmul_rn(x[16 * w + l], cs[16 * w + l]) : x[16 * w + l];
-                amax = fmaxf(amax, fabsf(v[l]));
-            }
+    const int lane = threadIdx.x & 63;
+    const uint64_t wave = (uint64_t)blockIdx.x * kEncodeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint64_t i0 = wave * kSuperUnroll; i0 < n_blocks; i0 += (uint64_t)gridDim.x * kEncodeWaves * kSuperUnroll) {
+        float v[kSuperUnroll][4];
+        load_super(src, col_scale, i0, n_blocks, blocks_per_row, lane, v);
+#pragma unroll
+        for (int u = 0; u < kSuperUnroll; ++u) {
+            if (i0 + u >= n_blocks) break;
+            float amax = fmaxf(fmaxf(fabsf(v[u][0]), fabsf(v[u][1])), fmaxf(fabsf(v[u][2]), fabsf(v[u][3])));
+            amax = dpp_fmax<kDppQuadXor1>(amax);
+            amax = dpp_fmax<kDppQuadXor2>(amax);
             const uint32_t b = ((f32_to_f16_bits(amax) + 0x80u) >> 8) & 0xFFu;
-            const float s = (float)__builtin_bit_cast(_Float16, (uint16_t)(b << 8));
+            const float s = f16_bits_to_f32(b << 8);
+            float r[4];
+            rint_div4<true>(v[u], s != 0.0f ? s : 1.0f, r);
             uint32_t word = 0;
-            for (int l = 0; l < 16; ++l) {
-                const float t = s != 0.0f ? __fdiv_rn(v[l], s) : 0.0f;
-                const float q = fminf(fmaxf(rintf(__fadd_rn(__fmul_rn(t, 1.5f), 1.5f)), 0.0f), 3.0f);
-                word |= (uint32_t)q << (2 * l);
+#pragma unroll
+            for (int q = 0; q < 4; ++q)  // s == 0: t = 0, code rint(1.5) = 2
+                word |= (s != 0.0f ? (uint32_t)fminf(fmaxf(r[q], 0.0f), 3.0f) : 2u) << (2 * q);
+            word <<= 8 * (lane & 3);
+            word |= dpp_u32<kDppQuadXor1>(word);
+            word |= dpp_u32<kDppQuadXor2>(word);
+            if ((lane & 3) == 0) {
+                uint8_t* blk = dst + 80 * (i0 + u);
+                reinterpret_cast<uint32_t*>(blk)[lane >> 2] = word;
+                blk[64 + (lane >> 2)] = (uint8_t)b;
             }
-            words[w] = word;
-            sb[w >> 2] |= b << (8 * (w & 3));
         }
-        uint4_t* o = reinterpret_cast<uint4_t*>(dst + 80 * i);  // 80-byte blocks: 16-byte aligned
-        for (int q = 0; q < 4; ++q) o[q] = uint4_t{words[4 * q], words[4 * q + 1], words[4 * q + 2], words[4 * q + 3]};
-        o[4] = uint4_t{sb[0], sb[1], sb[2], sb[3]};
     }
 }
 
+// One thread per q8_0 block: d = max|x| / 127, q = round_half_away(x * (1/d)).
 __global__ __launch_bounds__(kEncodeThreads) void q8_0_quantize_kernel(const float* __restrict__ src,
                                                                        const float* __restrict__ col_scale,
                                                                        uint8_t* __restrict__ dst, uint64_t n_blocks,
@@ -137,9 +213,13 @@ __global__ __launch_bounds__(kEncodeThreads) void q8_0_quantize_kernel(const flo
             v[4 * j + 3] = t.w;
         }
         if (col_scale) {
-            const float* cs = col_scale + 32u * (uint32_t)(i % blocks_per_row);
+            const float* cs = col_scale + 32u * mod_u64(i, blocks_per_row);
 #pragma unroll
-            for (int j = 0; j < 32; ++j) v[j] = __fmul_rn(v[j], cs[j]);
+            for (int j = 0; j < 8; ++j) {
+                const float4_t t = *reinterpret_cast<const float4_t*>(cs + 4 * j);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) v[4 * j + q] = __fmul_rn(v[4 * j + q], t[q]);
+            }
         }
         float amax = 0.0f;
 #pragma unroll
@@ -164,7 +244,7 @@ __global__ __launch_bounds__(kEncodeThreads) void q8_0_quantize_kernel(const flo
     }
 }
 
-// One thread per Q4_K (Q5_K) super-block (256 columns, 8 sub-blocks of 32),
+// Q4_K (Q5_K) super-blocks (256 columns, 8 sub-blocks of 32: 8 lanes each),
 // with L = 15 (31) code levels:
 //   lo_j = min(min(x), 0), hi_j = max(x), scale_j = (hi_j - lo_j) / L, min_j = -lo_j
 //   d = fp16(max_j scale_j / 63), dmin = fp16(max_j min_j / 63)
@@ -183,140 +263,146 @@ __global__ __launch_bounds__(kEncodeThreads) void k_quantize_kernel(const float*
     constexpr float kLevels = Q5 ? 31.0f : 15.0f;
     constexpr int kBlockBytes = Q5 ? 176 : 144;
     constexpr int kQs = Q5 ? 48 : 16;
-    for (uint64_t i = (uint64_t)blockIdx.x * kEncodeThreads + threadIdx.x; i < n_blocks;
-         i += (uint64_t)gridDim.x * kEncodeThreads) {
-        const float* x = src + 256 * i;
-        const float* cs = col_scale ? col_scale + 256u * (uint32_t)(i % blocks_per_row) : nullptr;
-        float scale[8], mins[8];
-        for (int j = 0; j < 8; ++j) {
-            float lo = INFINITY, hi = -INFINITY;
-            for (int l = 0; l < 32; ++l) {
-                const float v = cs ? __fmul_rn(x[32 * j + l], cs[32 * j + l]) : x[32 * j + l];
-                lo = fminf(lo, v);
-                hi = fmaxf(hi, v);
+    const int lane = threadIdx.x & 63;
+    const int j = lane >> 3;  // the lane's sub-block
+    const uint64_t wave = (uint64_t)blockIdx.x * kEncodeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    for (uint64_t i0 = wave * kSuperUnroll; i0 < n_blocks; i0 += (uint64_t)gridDim.x * kEncodeWaves * kSuperUnroll) {
+        float v[kSuperUnroll][4];
+        load_super(src, col_scale, i0, n_blocks, blocks_per_row, lane, v);
+        // lo and hi of each sub-block over its 8 lanes; lane l then keeps those
+        // of super-block l % 4, so the sub-block arithmetic (five divides) runs
+        // once for the four super-blocks
+        static_assert(kSuperUnroll == 4, "one lane of a quad per super-block");
+        float lo_u = 0.0f, hi_u = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kSuperUnroll; ++u) {
+            float lo = fminf(fminf(v[u][0], v[u][1]), fminf(v[u][2], v[u][3]));
+            float hi = fmaxf(fmaxf(v[u][0], v[u][1]), fmaxf(v[u][2], v[u][3]));
+            lo = dpp_fmin<kDppRowHalfMirror>(dpp_fmin<kDppQuadXor2>(dpp_fmin<kDppQuadXor1>(lo)));
+            hi = dpp_fmax<kDppRowHalfMirror>(dpp_fmax<kDppQuadXor2>(dpp_fmax<kDppQuadXor1>(hi)));
+            lo_u = (lane & 3) == u ? lo : lo_u;
+            hi_u = (lane & 3) == u ? hi : hi_u;
+        }
+        lo_u = fminf(lo_u, 0.0f);
+        const float scale = __fdiv_rn(__fsub_rn(hi_u, lo_u), kLevels);
+        const float mins = -lo_u;
+        float smax = scale, mmax = mins;
+#pragma unroll
+        for (int o = 8; o < 64; o <<= 1) {
+            smax = fmaxf(smax, __shfl_xor(smax, o));
+            mmax = fmaxf(mmax, __shfl_xor(mmax, o));
+        }
+        const uint32_t d_bits_u = f32_to_f16_bits(__fdiv_rn(smax, 63.0f));
+        const uint32_t dmin_bits_u = f32_to_f16_bits(__fdiv_rn(mmax, 63.0f));
+        const float df = f16_bits_to_f32(d_bits_u);
+        const float dminf = f16_bits_to_f32(dmin_bits_u);
+        const float a = (df != 0.0f) ? rintf(__fdiv_rn(scale, df)) : 0.0f;
+        const float m = (dminf != 0.0f) ? rintf(__fdiv_rn(mins, dminf)) : 0.0f;
+        const uint32_t sc_u = (uint32_t)fminf(fmaxf(a, 0.0f), 63.0f);
+        const uint32_t mq_u = (uint32_t)fminf(fmaxf(m, 0.0f), 63.0f);
+        const float step_u = __fmul_rn(df, (float)sc_u);
+        const float offs_u = __fmul_rn(dminf, (float)mq_u);
+        const uint32_t both_u = sc_u | (mq_u << 8), dd_u = d_bits_u | (dmin_bits_u << 16);
+#pragma unroll
+        for (int u = 0; u < kSuperUnroll; ++u) {
+            if (i0 + u >= n_blocks) break;
+            const int from = (lane & ~3) | u;  // this sub-block's lane of super-block u
+            const float step = __shfl(step_u, from), offs = __shfl(offs_u, from);
+            float n[4], r[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) n[q] = __fadd_rn(v[u][q], offs);
+            rint_div4<false>(n, step != 0.0f ? step : 1.0f, r);
+            uint32_t code = 0;  // the lane's four codes, one per byte
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                code |= (step != 0.0f ? (uint32_t)fminf(fmaxf(r[q], 0.0f), kLevels) : 0u) << (8 * q);
+            uint8_t* blk = dst + kBlockBytes * (i0 + u);  // 144- or 176-byte blocks: 16-byte aligned
+            // nibbles: sub-blocks 2c and 2c + 1 are 8 lanes apart
+            const uint32_t other = (uint32_t)__shfl_xor((int)code, 8);
+            if ((lane & 8) == 0)
+                reinterpret_cast<uint32_t*>(blk + kQs)[8 * (lane >> 4) + (lane & 7)] =
+                    (code & 0x0F0F0F0Fu) | ((other & 0x0F0F0F0Fu) << 4);
+            if constexpr (Q5) {  // qh: bit j of byte l, over the eight sub-blocks
+                uint32_t qh = ((code >> 4) & 0x01010101u) << j;
+#pragma unroll
+                for (int o = 8; o < 64; o <<= 1) qh |= (uint32_t)__shfl_xor((int)qh, o);
+                if (lane < 8) reinterpret_cast<uint32_t*>(blk + 16)[lane] = qh;
             }
-            lo = fminf(lo, 0.0f);
-            scale[j] = __fdiv_rn(__fsub_rn(hi, lo), kLevels);
-            mins[j] = -lo;
-        }
-        float smax = scale[0], mmax = mins[0];
-        for (int j = 1; j < 8; ++j) {
-            smax = fmaxf(smax, scale[j]);
-            mmax = fmaxf(mmax, mins[j]);
-        }
-        const uint32_t d_bits = f32_to_f16_bits(__fdiv_rn(smax, 63.0f));
-        const uint32_t dmin_bits = f32_to_f16_bits(__fdiv_rn(mmax, 63.0f));
-        const float df = f16_bits_to_f32(d_bits);
-        const float dminf = f16_bits_to_f32(dmin_bits);
-        uint32_t sc[8], mq[8];
-        float step[8], offs[8];
-        for (int j = 0; j < 8; ++j) {
-            const float a = (df != 0.0f) ? rintf(__fdiv_rn(scale[j], df)) : 0.0f;
-            const float m = (dminf != 0.0f) ? rintf(__fdiv_rn(mins[j], dminf)) : 0.0f;
-            sc[j] = (uint32_t)fminf(fmaxf(a, 0.0f), 63.0f);
-            mq[j] = (uint32_t)fminf(fmaxf(m, 0.0f), 63.0f);
-            step[j] = __fmul_rn(df, (float)sc[j]);
-            offs[j] = __fmul_rn(dminf, (float)mq[j]);
-        }
-        uint8_t* blk = dst + kBlockBytes * i;  // 144- or 176-byte blocks: 16-byte aligned
-        uint32_t head[4];
-        head[0] = d_bits | (dmin_bits << 16);
-        uint8_t scales[12];
-        for (int j = 0; j < 4; ++j) {
-            scales[j] = (uint8_t)((sc[j] & 63) | ((sc[j + 4] >> 4) << 6));
-            scales[j + 4] = (uint8_t)((mq[j] & 63) | ((mq[j + 4] >> 4) << 6));
-            scales[j + 8] = (uint8_t)((sc[j + 4] & 0xF) | ((mq[j + 4] & 0xF) << 4));
-        }
-        for (int w = 0; w < 3; ++w)
-            head[1 + w] = (uint32_t)scales[4 * w] | ((uint32_t)scales[4 * w + 1] << 8) |
-                          ((uint32_t)scales[4 * w + 2] << 16) | ((uint32_t)scales[4 * w + 3] << 24);
-        *reinterpret_cast<uint4_t*>(blk) = uint4_t{head[0], head[1], head[2], head[3]};
-        uint32_t qh[8] = {0, 0, 0, 0, 0, 0, 0, 0};  // Q5_K: 32 bytes
-        for (int c = 0; c < 4; ++c) {
-            for (int l4 = 0; l4 < 32; l4 += 16) {
-                uint32_t packed[4] = {0, 0, 0, 0};
-                for (int l = 0; l < 16; ++l) {
-                    uint32_t nib[2];
-                    for (int h = 0; h < 2; ++h) {
-                        const int j = 2 * c + h;
-                        const int e = 32 * j + l4 + l;
-                        const float v = cs ? __fmul_rn(x[e], cs[e]) : x[e];
-                        const float qf = (step[j] != 0.0f) ? __fdiv_rn(__fadd_rn(v, offs[j]), step[j]) : 0.0f;
-                        const uint32_t q = (uint32_t)fminf(fmaxf(rintf(qf), 0.0f), kLevels);
-                        nib[h] = q & 15u;
-                        if (Q5) qh[(l4 + l) >> 2] |= ((q >> 4) << j) << (8 * ((l4 + l) & 3));
-                    }
-                    packed[l >> 2] |= (nib[0] | (nib[1] << 4)) << (8 * (l & 3));
-                }
-                *reinterpret_cast<uint4_t*>(blk + kQs + 32 * c + l4) =
-                    uint4_t{packed[0], packed[1], packed[2], packed[3]};
-            }
-        }
-        if (Q5) {
-            *reinterpret_cast<uint4_t*>(blk + 16) = uint4_t{qh[0], qh[1], qh[2], qh[3]};
-            *reinterpret_cast<uint4_t*>(blk + 32) = uint4_t{qh[4], qh[5], qh[6], qh[7]};
+            // header: lane q < 4 holds scale bytes q, q + 4 and q + 8
+            const uint32_t lo_j = (uint32_t)__shfl((int)both_u, 8 * (lane & 3) + u);
+            const uint32_t hi_j = (uint32_t)__shfl((int)both_u, 8 * (lane & 3) + 32 + u);
+            const uint32_t dd = (uint32_t)__shfl((int)dd_u, u);
+            const uint32_t s0 = lo_j & 63u, m0 = lo_j >> 8, s1 = hi_j & 63u, m1 = hi_j >> 8;
+            uint32_t w0 = (s0 | ((s1 >> 4) << 6)) << (8 * (lane & 3));
+            uint32_t w1 = (m0 | ((m1 >> 4) << 6)) << (8 * (lane & 3));
+            uint32_t w2 = ((s1 & 15u) | ((m1 & 15u) << 4)) << (8 * (lane & 3));
+            w0 |= dpp_u32<kDppQuadXor1>(w0);
+            w1 |= dpp_u32<kDppQuadXor1>(w1);
+            w2 |= dpp_u32<kDppQuadXor1>(w2);
+            w0 |= dpp_u32<kDppQuadXor2>(w0);
+            w1 |= dpp_u32<kDppQuadXor2>(w1);
+            w2 |= dpp_u32<kDppQuadXor2>(w2);
+            if (lane == 0) *reinterpret_cast<uint4_t*>(blk) = uint4_t{dd, w0, w1, w2};
         }
     }
 }
 
-// One thread per Q6_K super-block (256 columns, 16 sub-blocks of 16), the
-// statement of oracle q6_k_quantize:
+// Q6_K super-blocks (256 columns, 16 sub-blocks of 16: one quad of lanes each),
+// the statement of oracle q6_k_quantize:
 //   sub_s = max|x| / 31, d = fp16(max_s sub_s / 127), sc_s = clip(rint(sub_s / d), 0, 127)
 //   q = clip(rint(x / (d * sc_s)), -32, 31) + 32
 // stored as ggml lays Q6_K out (qw35_types.metal:17-22): element
 // 128h + 32g + l has its low nibble in ql[64h + 32(g&1) + l] (high nibble for
 // g >= 2) and its top two bits at bit 2g of qh[32h + l].  Super-blocks are
-// 210 bytes (2-byte aligned), so the bytes are stored one at a time.
+// 210 bytes (2-byte aligned), so a word leaves as two 16-bit stores.
 __global__ __launch_bounds__(kEncodeThreads) void q6_k_quantize_kernel(const float* __restrict__ src,
                                                                        const float* __restrict__ col_scale,
                                                                        uint8_t* __restrict__ dst, uint64_t n_blocks,
                                                                        uint32_t blocks_per_row) {
-    for (uint64_t i = (uint64_t)blockIdx.x * kEncodeThreads + threadIdx.x; i < n_blocks;
-         i += (uint64_t)gridDim.x * kEncodeThreads) {
-        const float* x = src + 256 * i;
-        const float* cs = col_scale ? col_scale + 256u * (uint32_t)(i % blocks_per_row) : nullptr;
-        auto val = [&](int e) { return cs ? __fmul_rn(x[e], cs[e]) : x[e]; };
-        float sub[16];
-        float smax = 0.0f;
+    const int lane = threadIdx.x & 63;
+    const uint64_t wave = (uint64_t)blockIdx.x * kEncodeWaves + __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    auto store4 = [](uint8_t* p, uint32_t w) {
+        reinterpret_cast<uint16_t*>(p)[0] = (uint16_t)w;
+        reinterpret_cast<uint16_t*>(p)[1] = (uint16_t)(w >> 16);
+    };
+    for (uint64_t i0 = wave * kSuperUnroll; i0 < n_blocks; i0 += (uint64_t)gridDim.x * kEncodeWaves * kSuperUnroll) {
+        float v[kSuperUnroll][4];
+        load_super(src, col_scale, i0, n_blocks, blocks_per_row, lane, v);
 #pragma unroll
-        for (int sb = 0; sb < 16; ++sb) {
-            float amax = 0.0f;
-            for (int l = 0; l < 16; ++l) amax = fmaxf(amax, fabsf(val(16 * sb + l)));
-            sub[sb] = __fdiv_rn(amax, 31.0f);
-            smax = fmaxf(smax, sub[sb]);
-        }
-        const uint32_t d_bits = f32_to_f16_bits(__fdiv_rn(smax, 127.0f));
-        const float df = f16_bits_to_f32(d_bits);
-        float step[16];
-        uint8_t* blk = dst + 210 * i;
+        for (int u = 0; u < kSuperUnroll; ++u) {
+            if (i0 + u >= n_blocks) break;
+            float amax = fmaxf(fmaxf(fabsf(v[u][0]), fabsf(v[u][1])), fmaxf(fabsf(v[u][2]), fabsf(v[u][3])));
+            amax = dpp_fmax<kDppQuadXor1>(amax);
+            amax = dpp_fmax<kDppQuadXor2>(amax);
+            const float sub = __fdiv_rn(amax, 31.0f);
+            float smax = sub;
 #pragma unroll
-        for (int sb = 0; sb < 16; ++sb) {
-            const float a = (df != 0.0f) ? rintf(__fdiv_rn(sub[sb], df)) : 0.0f;
+            for (int o = 4; o < 64; o <<= 1) smax = fmaxf(smax, __shfl_xor(smax, o));
+            const uint32_t d_bits = f32_to_f16_bits(__fdiv_rn(smax, 127.0f));
+            const float df = f16_bits_to_f32(d_bits);
+            const float a = (df != 0.0f) ? rintf(__fdiv_rn(sub, df)) : 0.0f;
             const float scq = fminf(fmaxf(a, 0.0f), 127.0f);
-            step[sb] = __fmul_rn(df, scq);
-            blk[192 + sb] = (uint8_t)(int)scq;
-        }
-        auto code = [&](int e) {
-            const float st = step[e >> 4];
-            const float qf = (st != 0.0f) ? rintf(__fdiv_rn(val(e), st)) : 0.0f;
-            return (uint32_t)(int)(fminf(fmaxf(qf, -32.0f), 31.0f) + 32.0f);
-        };
+            const float step = __fmul_rn(df, scq);
+            float r[4];
+            rint_div4<false>(v[u], step != 0.0f ? step : 1.0f, r);
+            uint32_t code = 0;  // the lane's four codes, one per byte
 #pragma unroll
-        for (int j = 0; j < 128; ++j) {
-            const int h = j >> 6, gp = (j >> 5) & 1, l = j & 31;
-            const int e = 128 * h + 32 * gp + l;
-            blk[j] = (uint8_t)((code(e) & 15u) | ((code(e + 64) & 15u) << 4));
+            for (int q = 0; q < 4; ++q) {
+                const float qf = step != 0.0f ? r[q] : 0.0f;
+                code |= (uint32_t)(int)(fminf(fmaxf(qf, -32.0f), 31.0f) + 32.0f) << (8 * q);
+            }
+            uint8_t* blk = dst + 210 * (i0 + u);
+            // lane = 32h + 8g + l / 4: groups g and g + 2 share the bytes of ql, all four those of qh
+            const int h = lane >> 5, g = (lane >> 3) & 3, l = 4 * (lane & 7);
+            const uint32_t other = (uint32_t)__shfl_xor((int)code, 16);
+            uint32_t qh = ((code >> 4) & 0x03030303u) << (2 * g);
+            qh |= (uint32_t)__shfl_xor((int)qh, 8);
+            qh |= (uint32_t)__shfl_xor((int)qh, 16);
+            if (g < 2) store4(blk + 64 * h + 32 * g + l, (code & 0x0F0F0F0Fu) | ((other & 0x0F0F0F0Fu) << 4));
+            if (g == 2) store4(blk + 128 + 32 * h + l, qh);
+            if ((lane & 3) == 0) blk[192 + (lane >> 2)] = (uint8_t)(int)scq;
+            if (lane == 1) *reinterpret_cast<uint16_t*>(blk + 208) = (uint16_t)d_bits;
         }
-#pragma unroll
-        for (int j = 0; j < 64; ++j) {
-            const int h = j >> 5, l = j & 31;
-            uint32_t b = 0;
-#pragma unroll
-            for (int g = 0; g < 4; ++g) b |= (code(128 * h + 32 * g + l) >> 4) << (2 * g);
-            blk[128 + j] = (uint8_t)b;
-        }
-        blk[208] = (uint8_t)(d_bits & 0xFFu);
-        blk[209] = (uint8_t)(d_bits >> 8);
     }
 }
 
@@ -336,13 +422,19 @@ __global__ __launch_bounds__(kEncodeThreads) void f16_quantize_kernel(const floa
             v[4 + q] = b[q];
         }
         if (col_scale) {
-            const float* cs = col_scale + 8u * (uint32_t)(i % groups_per_row);
+            const float* cs = col_scale + 8u * mod_u64(i, groups_per_row);
 #pragma unroll
             for (int q = 0; q < 8; ++q) v[q] = __fmul_rn(v[q], cs[q]);
         }
         *reinterpret_cast<uint4_t*>(dst + 8 * i) =
             uint4_t{as_u32(h2(v[0], v[1])), as_u32(h2(v[2], v[3])), as_u32(h2(v[4], v[5])), as_u32(h2(v[6], v[7]))};
     }
+}
+
+// Blocks for n super-blocks, one wave per kSuperUnroll of them at a time.
+unsigned grid_for_super(uint64_t n) {
+    const uint64_t g = (n + kEncodeWaves * kSuperUnroll - 1) / (kEncodeWaves * kSuperUnroll);
+    return (unsigned)(g < (uint64_t)kEncodeBlocks ? g : (uint64_t)kEncodeBlocks);
 }
 
 unsigned grid_for(uint64_t n) {
@@ -376,25 +468,25 @@ hipError_t launch_quantize(uint32_t type_id, const float* src, int rows, int k, 
         }
         case kTypeQ6_K: {
             const uint64_t n = r * (uint64_t)(k / 256);
-            hipLaunchKernelGGL(q6_k_quantize_kernel, dim3(grid_for(n)), dim3(kEncodeThreads), 0, stream, src,
+            hipLaunchKernelGGL(q6_k_quantize_kernel, dim3(grid_for_super(n)), dim3(kEncodeThreads), 0, stream, src,
                                col_scale, static_cast<uint8_t*>(dst), n, (uint32_t)(k / 256));
             break;
         }
         case kTypeGF2: {
             const uint64_t n = r * (uint64_t)(k / 256);
-            hipLaunchKernelGGL(gf2_pack_kernel, dim3(grid_for(n)), dim3(kEncodeThreads), 0, stream, src, col_scale,
+            hipLaunchKernelGGL(gf2_pack_kernel, dim3(grid_for_super(n)), dim3(kEncodeThreads), 0, stream, src, col_scale,
                                static_cast<uint8_t*>(dst), n, (uint32_t)(k / 256));
             break;
         }
         case kTypeQ5_K: {
             const uint64_t n = r * (uint64_t)(k / 256);
-            hipLaunchKernelGGL(k_quantize_kernel<true>, dim3(grid_for(n)), dim3(kEncodeThreads), 0, stream, src,
+            hipLaunchKernelGGL(k_quantize_kernel<true>, dim3(grid_for_super(n)), dim3(kEncodeThreads), 0, stream, src,
                                col_scale, static_cast<uint8_t*>(dst), n, (uint32_t)(k / 256));
             break;
         }
         default: {
             const uint64_t n = r * (uint64_t)(k / 256);
-            hipLaunchKernelGGL(k_quantize_kernel<false>, dim3(grid_for(n)), dim3(kEncodeThreads), 0, stream, src,
+            hipLaunchKernelGGL(k_quantize_kernel<false>, dim3(grid_for_super(n)), dim3(kEncodeThreads), 0, stream, src,
                                col_scale, static_cast<uint8_t*>(dst), n, (uint32_t)(k / 256));
             break;
         }

@@ -1,0 +1,38 @@
+"""The wave-per-super-block encoders (GF2, Q4_K, Q5_K, Q6_K) at the edges of
+their grid, bit for bit against the oracle: fewer super-blocks than one wave
+takes at a time, a count that is not a multiple of it, and more than one round
+of the launch's fixed grid (2048 blocks of 4 waves of 4 super-blocks)."""
+from __future__ import annotations
+
+import numpy as np
+import pytest
+
+from oracle import matvec as om
+from oracle import q6_k as oq6
+from tests.helpers import awq_scales
+
+pytestmark = pytest.mark.gpu
+
+CODECS = {"gf2": om.TYPE_GF2, "q4_k": om.TYPE_Q4_K, "q5_k": om.TYPE_Q5_K, "q6_k": om.TYPE_Q6_K}
+
+
+@pytest.mark.parametrize("name", list(CODECS))
+@pytest.mark.parametrize("rows,k,scaled", [(3, 256, False), (7, 768, True), (2051, 4096, True)])
+def test_super_block_encoders_bit_exact(cuda, name, rows, k, scaled):
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    rng = np.random.default_rng(rows)
+    w = (rng.standard_normal((rows, k)) * 0.02 * np.exp2(rng.uniform(-12, 6, (rows, 1)))).astype(np.float32)
+    w[0, 16:80] = 0.0
+    w[1, :256] = np.abs(w[1, :256])  # no negative minimum
+    w[2, :256] = -np.abs(w[2, :256])
+    w[-2, -256:] = (np.arange(256) % 31 - 8) * 0.5  # quotients on and beside ties
+    w[-1, -256:] = 0.0
+    s = awq_scales(rng, k) if scaled else None
+    got = rt.quantize(torch.from_numpy(w).to(cuda), CODECS[name],
+                      col_scale=torch.from_numpy(s).to(cuda) if scaled else None)
+    v = (w * s[None, :]).astype(np.float32) if scaled else w
+    want = oq6.q6_k_quantize(v) if name == "q6_k" else om.quantize(CODECS[name], v)
+    assert np.array_equal(got.cpu().numpy().reshape(rows, -1), np.asarray(want).reshape(rows, -1).view(np.uint8))
