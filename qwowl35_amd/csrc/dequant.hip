@@ -20,6 +20,8 @@
 namespace qw35 {
 namespace {
 
+typedef uint32_t uint2_t __attribute__((ext_vector_type(2)));
+
 __device__ __forceinline__ float f16_to_f32(uint32_t bits16) {
     return (float)__builtin_bit_cast(_Float16, (uint16_t)bits16);
 }
@@ -91,33 +93,35 @@ __global__ __launch_bounds__(256) void dequant_kernel(uint32_t type_id, const ui
             const uint32_t hi = (blk[128 + 32 * h + l] >> (2 * gg)) & 3u;
             v[i] = dsc * (float)((int)(lo | (hi << 4)) - 32);
         }
-    } else {  // Q4_K, Q5_K
+    } else {  // Q4_K, Q5_K: 16-byte aligned blocks; header, codes and high bits as one vector load each
+        // (byte loads took 44 / 65 us for the fp16 image of 12288x4096, 2.9 / 2.1 TB/s)
         const bool q5 = type_id == kTypeQ5_K;
         const size_t bb = q5 ? 176 : 144;
-        const uint8_t* row = w + src_row * (size_t)(k >> 8) * bb;
         const int col = 8 * g;
-        const uint8_t* blk = row + (size_t)(col >> 8) * bb;
+        const uint8_t* blk = w + src_row * (size_t)(k >> 8) * bb + (size_t)(col >> 8) * bb;
         const int e = col & 255;
         const int j = e >> 5;
-        const uint8_t* sc = blk + 4;
+        const uint4_t hd = *reinterpret_cast<const uint4_t*>(blk);
+        const uint2_t qs = *reinterpret_cast<const uint2_t*>(blk + (q5 ? 48 : 16) + (j >> 1) * 32 + (e & 31));
+        uint2_t qh = {0u, 0u};
+        if (q5) qh = *reinterpret_cast<const uint2_t*>(blk + 16 + (e & 31));
+        const int sh = 8 * (j & 3);
         uint32_t s6, m6;
         if (j < 4) {
-            s6 = sc[j] & 63;
-            m6 = sc[j + 4] & 63;
+            s6 = (hd.y >> sh) & 63u;
+            m6 = (hd.z >> sh) & 63u;
         } else {
-            s6 = (sc[j + 4] & 0x0F) | ((sc[j - 4] >> 6) << 4);
-            m6 = (sc[j + 4] >> 4) | ((sc[j] >> 6) << 4);
+            const uint32_t t = hd.w >> sh;
+            s6 = (t & 0x0Fu) | (((hd.y >> sh) >> 6 & 3u) << 4);
+            m6 = ((t >> 4) & 0x0Fu) | (((hd.z >> sh) >> 6 & 3u) << 4);
         }
-        const float d = f16_to_f32((uint32_t)blk[0] | ((uint32_t)blk[1] << 8));
-        const float dmin = f16_to_f32((uint32_t)blk[2] | ((uint32_t)blk[3] << 8));
-        const float dsc = d * (float)s6;
-        const float mm = dmin * (float)m6;
-        const uint8_t* qs = blk + (q5 ? 48 : 16) + (j >> 1) * 32 + (e & 31);
-        const uint8_t* qh = blk + 16 + (e & 31);
+        const float dsc = f16_to_f32(hd.x & 0xFFFFu) * (float)s6;
+        const float mm = f16_to_f32(hd.x >> 16) * (float)m6;
 #pragma unroll
         for (int i = 0; i < 8; ++i) {
-            uint32_t q = (j & 1) ? (qs[i] >> 4) : (qs[i] & 0x0F);
-            if (q5) q |= ((qh[i] >> j) & 1u) << 4;
+            const uint32_t qw = i < 4 ? qs.x : qs.y, hw = i < 4 ? qh.x : qh.y;
+            uint32_t q = (qw >> (8 * (i & 3) + 4 * (j & 1))) & 0x0Fu;
+            q |= ((hw >> (8 * (i & 3) + j)) & 1u) << 4;
             v[i] = dsc * (float)q - mm;
         }
     }
