@@ -206,9 +206,13 @@ struct KqLds {
     static constexpr int kActStride = 264;  // halves per activation row
     static constexpr int kAct = 2 * NB * kActStride * 2;
     static constexpr int kSx = (FMT == kFmtQ4K || FMT == kFmtQ5K) ? NB * 8 * 4 : 0;
+    // Batch 3..8: a chunk's activation operands move to registers once
+    // (32 VGPRs, shared by every row tile) before the first tile is
+    // transposed, so the two buffers share their bytes.
+    static constexpr bool kActRegs = NB >= 4;
     static constexpr int kXposeOff = 0;
-    static constexpr int kActOff = kXpose;
-    static constexpr int kZeroOff = kActOff + kAct;
+    static constexpr int kActOff = kActRegs ? 0 : kXpose;
+    static constexpr int kZeroOff = kActRegs ? (kXpose > kAct ? kXpose : kAct) : kActOff + kAct;
     static constexpr int kSxOff = kZeroOff + 128;
     static constexpr int kBytes = kSxOff + kSx;
 };
@@ -471,13 +475,31 @@ __device__ __forceinline__ void kq_gemv_body(GemvArgs args) {
                 const _Float16* arow =
                     a_live ? xs + (size_t)n * L::kActStride : reinterpret_cast<const _Float16*>(wblk + L::kZeroOff);
                 const int a_step = a_live ? 32 : 0;
-                // GF4: the chunk's activation operands, shared by every tile (words 8kq + j).
-                half8_t ga[FMT == kFmtGF4 ? 8 : 1];
+                if constexpr (L::kActRegs) wave_sync_lds();  // the staged rows, before other lanes read them
+                // The chunk's activation operands, shared by every tile: GF4 words
+                // 8kq + j; the other formats' 32-column blocks j (Q6_K: its
+                // 16-column sub-blocks) where they are held in registers.
+                half8_t ga[FMT == kFmtGF4 || (L::kActRegs && FMT != kFmtQ6K) ? 8 : 1];
+                half4_t ga6[L::kActRegs && FMT == kFmtQ6K ? 16 : 1];
                 if constexpr (FMT == kFmtGF4) {
                     const _Float16* ap = a_live ? arow + 64 * kq : arow;
 #pragma unroll
                     for (int j = 0; j < 8; ++j) ga[j] = *reinterpret_cast<const half8_t*>(ap + (a_live ? 8 * j : 0));
+                } else if constexpr (L::kActRegs && FMT == kFmtQ6K) {
+                    const _Float16* ap = a_live ? arow + 4 * kq : arow;
+#pragma unroll
+                    for (int j = 0; j < 16; ++j)
+                        ga6[j] = *reinterpret_cast<const half4_t*>(ap + (a_live ? 16 * j : 0));
+                } else if constexpr (L::kActRegs) {
+#pragma unroll
+                    for (int j = 0; j < 8; ++j) ga[j] = *reinterpret_cast<const half8_t*>(arow + a_step * j + 8 * kq);
                 }
+                auto a_op = [&](int j) -> half8_t {
+                    if constexpr (L::kActRegs) return ga[j];
+                    else return *reinterpret_cast<const half8_t*>(arow + a_step * j + 8 * kq);
+                };
+                // the transposes below reuse the activation buffer's bytes
+                if constexpr (L::kActRegs) wave_sync_lds();
 
 #pragma unroll
                 for (int t = 0; t < RT; ++t) {
@@ -527,7 +549,7 @@ __device__ __forceinline__ void kq_gemv_body(GemvArgs args) {
                                 s8x4_to_h(d0, bias, b4[0], b4[1]);
                                 s8x4_to_h(d1, bias, b4[2], b4[3]);
                                 const half8_t bop = __builtin_bit_cast(half8_t, uint4_t{b4[0], b4[1], b4[2], b4[3]});
-                                const half8_t aop = *reinterpret_cast<const half8_t*>(arow + a_step * j + 8 * kq);
+                                const half8_t aop = a_op(j);
                                 const float4_t dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(
                                     aop, bop, float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                                 cs0 = __builtin_fmaf(dsc, dd[0] + dd[1], cs0);
@@ -564,7 +586,7 @@ __device__ __forceinline__ void kq_gemv_body(GemvArgs args) {
                                         __builtin_elementwise_fma(pq, h2(0.25f, 0.25f), h2(-256.75f, -256.75f)) * s2);
                                 }
                                 const half8_t bop = __builtin_bit_cast(half8_t, uint4_t{b4[0], b4[1], b4[2], b4[3]});
-                                const half8_t aop = *reinterpret_cast<const half8_t*>(arow + a_step * j + 8 * kq);
+                                const half8_t aop = a_op(j);
                                 dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, bop, dd, 0, 0, 0);
                             }
                             constexpr float kFourThirds = 4.0f / 3.0f;
@@ -610,7 +632,9 @@ __device__ __forceinline__ void kq_gemv_body(GemvArgs args) {
                                         uint32_t b0, b1;
                                         u4x4_to_h(qv, bias, b0, b1);
                                         const half4_t bop = __builtin_bit_cast(half4_t, uint2_t_{b0, b1});
-                                        const half4_t aop = *reinterpret_cast<const half4_t*>(abase + astep * sbk);
+                                        half4_t aop;
+                                        if constexpr (L::kActRegs) aop = ga6[sbk];
+                                        else aop = *reinterpret_cast<const half4_t*>(abase + astep * sbk);
                                         dd[u] = __builtin_amdgcn_mfma_f32_16x16x16f16(
                                             aop, bop, float4_t{0.f, 0.f, 0.f, 0.f}, 0, 0, 0);
                                     }
@@ -701,7 +725,7 @@ __device__ __forceinline__ void kq_gemv_body(GemvArgs args) {
                                         as_half2(__builtin_amdgcn_perm(ebase, t1, 0x04030402u)), s2, n2));
                                     const half8_t bop =
                                         __builtin_bit_cast(half8_t, uint4_t{b4[0], b4[1], b4[2], b4[3]});
-                                    const half8_t aop = *reinterpret_cast<const half8_t*>(arow + a_step * j + 8 * kq);
+                                    const half8_t aop = a_op(j);
                                     dd = __builtin_amdgcn_mfma_f32_16x16x32_f16(aop, bop, dd, 0, 0, 0);
                                 }
                             }
@@ -894,38 +918,70 @@ struct KqPlan {
 // Q6_K {1, 8, 2, 2} 175 us ({2, 16, 1, 1} 183 us; now two tiles, below), GF2
 // {3, 8, 2, 2} 113 us ({2, 16, 1, 1} 119 us); Q5_K keeps {2, 16, 1, 1} 157 us
 // ({3, 8, 2, 2} 160 us).
-inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false) {
+inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, bool swiglu = false) {
     const int chunks = k >> 8;
     const int tiles = (rows + 15) / 16;
-    // Batch 4..8, k = 12288, at most 256 row tiles (the 9B's down projection):
-    // with one tile per workgroup every workgroup would stage the whole
-    // activation batch, so K is split four ways across workgroups of four
-    // tiles, twelve waves, one chunk per wave (GF4 b8 13.0-13.7 us, Q4_K 15.7-16.4,
-    // against 17.9 / 21.0 unsplit; two-chunk waves or two-tile workgroups
-    // 14.6-22 us).  At k = 4096 no split beat the unsplit q8_0 launch.
-    if (split_ok && nb >= 4 && tiles <= 256 && chunks == 48) return {4, 12, 1, 1, 4};
+    if (nb >= 4) {
+        // Batch 3..8, k = 12288, at most 256 row tiles (the 9B's down projection):
+        // with one tile per workgroup every workgroup would stage the whole
+        // activation batch, so K is split four ways across workgroups of four
+        // tiles, twelve waves, one chunk per wave (b8, us, against the best
+        // unsplit plan: GF4 13.6 / 16.4, Q4_K 15.5 / 17.8, q8_0 19.4 / 19.5;
+        // two-chunk waves or two-tile workgroups 14.6-22).
+        if (split_ok && tiles <= 256 && chunks == 48) return {4, 12, 1, 1, 4};
+        // Longer rows of 257..384 tiles: three tiles and two splits keep one
+        // workgroup per CU (5120x17408 b8, us, against two unsplit tiles: GF4
+        // 22.6 / 25.1, Q4_K 24.9 / 27.3, Q5_K 27.5 / 30.5, GF2 22.8 / 26.9;
+        // q8_0 51 / 35.0).
+        if (split_ok && fmt != kFmtQ8 && tiles > 256 && tiles <= 384 && chunks > 48 && chunks % 2 == 0)
+            return {3, 12, 2, 1, 2};
+        if (chunks <= 4) return {1, 4, 1, 1};
+        if (tiles >= 4096 && chunks > 8 && chunks <= 16 && !swiglu) {
+            // LM-head sized: at batch 8 four tiles per 4-wave workgroup (head b8
+            // Q4_K 199 us, Q6_K 278, Q5_K 249, GF2 176; with {2, 4, 4, 2} 234 /
+            // 322 / 261 / 210 us); Q4_K eight tiles (one sweep on one box: 170.3
+            // us against 173.5 with four, 175.9 with six; Q6_K 258.7 with eight,
+            // 240.3 with four)
+            if (fmt == kFmtQ8) return {4, 8, 2, 1};
+            if (fmt == kFmtGF4) return {3, 8, 2, 1};
+            if (nb >= 8 && fmt == kFmtQ4K) return {8, 4, 4, 1};
+            return nb >= 8 ? KqPlan{4, 4, 4, 1} : KqPlan{2, 4, 4, 2};
+        }
+        // Otherwise as many row tiles per workgroup as leave one workgroup per
+        // CU: the launch's time is a fixed start and tail, plus per round of
+        // workgroups the staging of the batch and the tiles.  One sweep on one
+        // box over 2048..13824 rows, k = 2560..17408 and every codec (b8, us,
+        // the plan here against the next best tile count): 6144x4096 (two
+        // tiles) q8_0 10.9 / 13.2, Q4_K 9.6 / 12.3; 10240x7168 (three) q8_0
+        // 23.7 / 29.3, Q5_K 21.0 / 27.3; 4096x5120 (one) GF4 8.9 / 9.9;
+        // fused 9728x2560 (three) GF4 12.1 / 15.0; one tile at any row count
+        // took 1.3-2 times as long where it needs several rounds.
+        // One or two tiles run one chunk per wave up to 16 chunks (4096x4096 b8
+        // q8_0 9.2 -> 8.6 us, 8192x4096 11.9 -> 11.5), longer rows on twelve
+        // waves in rounds; more tiles hold eight waves' loads.
+        if (tiles <= 256)
+            return chunks <= 8 ? KqPlan{1, 8, 1, 1} : chunks > 12 && chunks <= 16 ? KqPlan{1, 16, 1, 1} : KqPlan{1, 12, 2, 1};
+        if (tiles <= 512) {
+            if (chunks <= 8) return {2, 8, 2, 1};
+            // (two fused tiles per wave spill at sixteen waves)
+            return chunks > 12 && chunks <= 16 && !swiglu ? KqPlan{2, 16, 1, 1} : KqPlan{2, 12, 2, 1};
+        }
+        if (tiles <= 768) {
+            // fused q8_0: its five loads per tile and matrix spill in rounds,
+            // and at batch 3..4 one tile per workgroup is faster (12288x4096
+            // 24.6 us against 28.4; at batch 8 34.1 against 29.1)
+            if (swiglu && fmt == kFmtQ8 && chunks > 16) return {2, 12, 2, 1};
+            if (swiglu && fmt == kFmtQ8 && nb < 8) return {1, 8, 2, 1};
+            return {3, 8, 2, 1};
+        }
+        if (swiglu) return {2, 12, 2, 1};
+        return {4, 8, 2, 1};
+    }
     // Longer rows: eight waves of four chunks per round (kq_mfma_gemv_long).
     if (chunks > 48) return {1, 8, 4, 2};
     if (chunks <= 4) return {1, 4, 1, 1};
     if (chunks <= 8) return {1, 8, 1, 1};
     if (chunks <= 16) {
-        if (nb >= 4) {
-            if (tiles >= 512) {
-                if (fmt != kFmtQ8 && fmt != kFmtGF4) {
-                    // LM-head sized: at batch 8 four tiles per 4-wave workgroup
-                    // (head b8 Q4_K 199 us, Q6_K 278, Q5_K 249, GF2 176; with
-                    // {2, 4, 4, 2} 234 / 322 / 261 / 210 us); Q4_K eight tiles
-                    // (one sweep on one box: 170.3 us against 173.5 with four,
-                    // 175.9 with six; Q6_K 258.7 with eight, 240.3 with four)
-                    if (tiles >= 4096 && nb >= 8 && fmt == kFmtQ4K) return {8, 4, 4, 1};
-                    if (tiles >= 4096) return nb >= 8 ? KqPlan{4, 4, 4, 1} : KqPlan{2, 4, 4, 2};
-                    return {4, 8, 2, 1};
-                }
-                if (fmt == kFmtQ8) return {4, 8, 2, 1};
-                return {3, 8, 2, 2};
-            }
-            return fmt == kFmtQ8 ? KqPlan{1, 8, 2, 1} : KqPlan{1, 8, 2, 2};
-        }
         if (tiles >= 4096) {  // LM-head sized
             if (fmt == kFmtQ4K) return {3, 8, 2, 2};
             // GF2 (cached loads): four tiles per 4-wave workgroup, one sweep on
@@ -940,9 +996,7 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false) {
         return {1, 8, 2, 2};
     }
     if (chunks <= 32) return {1, 8, 4, 2};
-    if (fmt != kFmtQ8 && fmt != kFmtGF4) return nb >= 4 ? KqPlan{1, 12, 4, 2} : KqPlan{1, 16, 3, 2};
-    // GF4 4096 x 12288 b8: {1, 12, 4, 2} 17.1 us ({1, 8, 6, 2} 17.9 us, two sweeps)
-    if (fmt == kFmtGF4 && nb >= 8) return {1, 12, 4, 2};
+    if (fmt != kFmtQ8 && fmt != kFmtGF4) return {1, 16, 3, 2};
     return {1, 8, 6, 2};
 }
 
@@ -1033,74 +1087,80 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
         total_rows = 0;
         for (int s = 0; s < a.n_seg; ++s) total_rows += a.seg_rows[s];
     }
-    if ((a.k >> 8) > 48)  // the long-row plan of plan_kq, in rounds of 32 chunks
-        return kq_launch_cfg<FMT, NB, 1, 8, 4, (kq_fits<FMT, NB, 1, 2, SWIGLU>() ? 2 : 1), SWIGLU, true>(a, stream);
-    KqPlan p = plan_kq(FMT, total_rows, a.k, NB, a.ks_ws != nullptr && !a.am_token);
+    KqPlan p = plan_kq(FMT, total_rows, a.k, NB, a.ks_ws != nullptr && !a.am_token, SWIGLU);
     if (p.s > 1) {
         int groups = (a.rows + 16 * p.rt - 1) / (16 * p.rt);
         if (a.n_seg > 1) {
             groups = 0;
             for (int s = 0; s < a.n_seg; ++s) groups += (a.seg_rows[s] + 16 * p.rt - 1) / (16 * p.rt);
         }
-        if (a.ks_ws_bytes < kq_split_ws_bytes(groups, p.s, p.rt, NB, SWIGLU ? 2 : 1))
-            p = plan_kq(FMT, total_rows, a.k, NB, false);
+        if (groups > kKsCounters || a.ks_ws_bytes < kq_split_ws_bytes(groups, p.s, p.rt, NB, SWIGLU ? 2 : 1))
+            p = plan_kq(FMT, total_rows, a.k, NB, false, SWIGLU);
     }
-    // Fused gate/up holds two matrices' loads per tile: more than two row tiles
-    // per workgroup spill registers, so those take the one-tile shape below.
 #define QW35_KQ_PLAN(RT, KS, CPW, P)                                                             \
-    if constexpr (kq_fits<FMT, NB, RT, P, SWIGLU>() && (!SWIGLU || RT <= 2)) {                     \
+    if constexpr (kq_fits<FMT, NB, RT, P, SWIGLU>()) {                                             \
         if (p.rt == RT && p.ks == KS && p.cpw == CPW && p.p == P)                                  \
             return kq_launch_cfg<FMT, NB, RT, KS, CPW, P, SWIGLU>(a, stream, p.s);                 \
     }
-    QW35_KQ_PLAN(1, 4, 1, 1)
-    QW35_KQ_PLAN(1, 8, 1, 1)
-    QW35_KQ_PLAN(1, 8, 2, 2)
-    QW35_KQ_PLAN(3, 8, 2, 2)
-    QW35_KQ_PLAN(4, 8, 2, 1)
-    QW35_KQ_PLAN(1, 8, 4, 2)
-    QW35_KQ_PLAN(1, 8, 6, 2)
-    if constexpr (FMT == kFmtQ8) {
-        if constexpr (NB >= 4) {
-            QW35_KQ_PLAN(1, 8, 2, 1)
+    if constexpr (NB >= 4) {
+        // the same plan in rounds where its waves do not cover the K slice
+#define QW35_KQ_ROUNDS(RT, KS, CPW, P)                                                           \
+    if constexpr (kq_fits<FMT, NB, RT, P, SWIGLU>()) {                                             \
+        if (p.rt == RT && p.ks == KS && p.cpw == CPW && p.p == P)                                  \
+            return (a.k >> 8) / p.s > KS * CPW                                                     \
+                       ? kq_launch_cfg<FMT, NB, RT, KS, CPW, P, SWIGLU, true>(a, stream, p.s)      \
+                       : kq_launch_cfg<FMT, NB, RT, KS, CPW, P, SWIGLU>(a, stream, p.s);           \
+    }
+        QW35_KQ_PLAN(1, 4, 1, 1)
+        QW35_KQ_PLAN(1, 8, 1, 1)
+        QW35_KQ_PLAN(1, 16, 1, 1)
+        QW35_KQ_ROUNDS(1, 12, 2, 1)
+        QW35_KQ_PLAN(2, 8, 2, 1)
+        QW35_KQ_ROUNDS(2, 12, 2, 1)
+        if constexpr (SWIGLU && FMT == kFmtQ8) {
+            QW35_KQ_PLAN(3, 8, 2, 1)
+            if constexpr (NB == 4) { QW35_KQ_PLAN(1, 8, 2, 1) }
         } else {
-            QW35_KQ_PLAN(1, 16, 1, 1)
+            QW35_KQ_ROUNDS(3, 8, 2, 1)
         }
-    }
-    if constexpr (NB == 8 && (FMT == kFmtQ4K || FMT == kFmtQ6K || FMT == kFmtQ5K || FMT == kFmtGF2)) {
-        QW35_KQ_PLAN(4, 4, 4, 1)
-    }
-    if constexpr (NB == 8 && FMT == kFmtQ4K) {
-        QW35_KQ_PLAN(8, 4, 4, 1)
-    }
-    if constexpr (NB <= 2 && FMT == kFmtQ6K) {
-        QW35_KQ_PLAN(2, 8, 2, 2)
-    }
-    if constexpr (NB <= 2 && FMT == kFmtGF2) {
-        QW35_KQ_PLAN(4, 4, 4, 1)
-    }
-    if constexpr (NB == 8 && FMT == kFmtGF4) {
-        QW35_KQ_PLAN(1, 12, 4, 2)
-    }
-    if constexpr (NB >= 4 && !SWIGLU) {  // the K-split plan
-        QW35_KQ_PLAN(4, 12, 1, 1)
-    }
-    if constexpr (FMT == kFmtQ4K || FMT == kFmtQ5K || FMT == kFmtQ6K || FMT == kFmtGF2) {
-        if constexpr (NB >= 4) {
-            QW35_KQ_PLAN(2, 4, 4, 2)
-            QW35_KQ_PLAN(1, 12, 4, 2)
-        } else {
+        if constexpr (!SWIGLU) {
             QW35_KQ_PLAN(2, 16, 1, 1)
+            QW35_KQ_ROUNDS(4, 8, 2, 1)
+            QW35_KQ_PLAN(4, 12, 1, 1)    // the K-split plans
+            QW35_KQ_ROUNDS(3, 12, 2, 1)
+            if constexpr (FMT == kFmtQ4K && NB == 8) { QW35_KQ_PLAN(8, 4, 4, 1) }
+            if constexpr (FMT != kFmtQ8 && FMT != kFmtGF4) {
+                if constexpr (NB == 8) {
+                    QW35_KQ_PLAN(4, 4, 4, 1)
+                } else {
+                    QW35_KQ_PLAN(2, 4, 4, 2)
+                }
+            }
+        }
+#undef QW35_KQ_ROUNDS
+    } else {
+        if ((a.k >> 8) > 48)  // the long-row plan, in rounds of 32 chunks
+            return kq_launch_cfg<FMT, NB, 1, 8, 4, (kq_fits<FMT, NB, 1, 2, SWIGLU>() ? 2 : 1), SWIGLU, true>(a, stream);
+        QW35_KQ_PLAN(1, 4, 1, 1)
+        QW35_KQ_PLAN(1, 8, 1, 1)
+        QW35_KQ_PLAN(1, 8, 2, 2)
+        QW35_KQ_PLAN(1, 8, 4, 2)
+        QW35_KQ_PLAN(1, 8, 6, 2)
+        if constexpr (FMT == kFmtQ8) { QW35_KQ_PLAN(1, 16, 1, 1) }
+        // Fused gate/up holds two matrices' loads per tile: more than two row
+        // tiles per workgroup spill registers, so those take the one-tile
+        // shape below.
+        if constexpr (FMT == kFmtQ4K && !SWIGLU) { QW35_KQ_PLAN(3, 8, 2, 2) }
+        if constexpr (FMT == kFmtQ6K) { QW35_KQ_PLAN(2, 8, 2, 2) }
+        if constexpr (FMT == kFmtGF2 && !SWIGLU) { QW35_KQ_PLAN(4, 4, 4, 1) }
+        if constexpr (FMT == kFmtQ5K) { QW35_KQ_PLAN(2, 16, 1, 1) }
+        if constexpr (FMT == kFmtQ4K || FMT == kFmtQ5K || FMT == kFmtQ6K || FMT == kFmtGF2) {
             QW35_KQ_PLAN(1, 16, 3, 2)
         }
+        // over the load budget or the register budget (fused gate/up): one tile per workgroup
+        if (p.rt > 1)
+            return kq_launch_cfg<FMT, NB, 1, 8, 2, (kq_fits<FMT, NB, 1, 2, SWIGLU>() ? 2 : 1), SWIGLU>(a, stream);
     }
-    // Fused gate/up planned with more than two tiles: three tiles with one
-    // chunk in flight (half the load registers of the planned shape, so no
-    // spills); 12288 rows are then exactly 256 workgroups, one per CU.
-    if constexpr (SWIGLU && NB >= 4 && kq_fits<FMT, NB, 3, 1, SWIGLU>()) {
-        if (p.rt > 2) return kq_launch_cfg<FMT, NB, 3, 8, 2, 1, SWIGLU>(a, stream);
-    }
-    // over the load budget or the register budget (fused gate/up): one tile per workgroup
-    if (p.rt > 1) return kq_launch_cfg<FMT, NB, 1, 8, 2, (kq_fits<FMT, NB, 1, 2, SWIGLU>() ? 2 : 1), SWIGLU>(a, stream);
 #undef QW35_KQ_PLAN
     return hipErrorInvalidValue;
 }

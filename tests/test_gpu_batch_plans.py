@@ -1,0 +1,86 @@
+"""The batch 3..8 GEMV plans at the edges where the row-tile count per workgroup
+or the wave count changes: 256 / 512 / 768 row tiles of 16, 8 / 12 / 16 / 24 and
+48 chunks of 256 columns, and the K split of longer rows.  Each output against
+an fp64 product of the library's dequantised weights (bit-exact against the
+oracle in the other tests) within 1e-6 relative L2 plus, for GF2's thirds and
+the fp16 hi/lo activations, their 2^-22: 2e-6."""
+from __future__ import annotations
+
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+TYPES = {"gf4": 100, "gf2": 101, "q8_0": 8, "q4_k": 12, "q5_k": 13, "q6_k": 14}
+# rows, k, the plan's (row tiles, waves) for a plain GEMV at batch 3..8
+SHAPES = [(4096, 1536, (1, 8)), (4096, 2560, (1, 12)), (4088, 3584, (1, 16)), (1000, 5120, (1, 12)),
+          (4104, 1536, (2, 8)), (4104, 2560, (2, 12)), (8192, 3584, (2, 16)), (4104, 5120, (2, 12)),
+          (8200, 2560, (3, 8)), (12288, 5120, (3, 8)), (12296, 1536, (4, 8)), (12296, 5120, (4, 8))]
+
+
+def _weight(name, rows, k, seed):
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    g = torch.Generator(device="cuda")
+    g.manual_seed(seed)
+    return rt.quantize_weight(torch.randn((rows, k), generator=g, device="cuda") * 0.02, TYPES[name])
+
+
+def _close(y, want):
+    err = float((y.double() - want).norm() / want.norm())
+    assert err <= 2e-6, err
+
+
+@pytest.mark.parametrize("nb", [3, 8])
+@pytest.mark.parametrize("name", list(TYPES))
+@pytest.mark.parametrize("rows,k,plan", SHAPES)
+def test_batch_plans(cuda, name, rows, k, plan, nb):
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    w = _weight(name, rows, k, rows + nb)
+    kernel, args = rt.gemv_kernel(w, nb)["name"].split("<")
+    if kernel != "gf4_mfma_gemv":  # (GF4 whose staged batch fits LDS runs its own kernel)
+        assert tuple(int(v) for v in args.split(",")[2:4]) == plan, args
+    x = torch.randn((nb, k), device=cuda)
+    awq = torch.rand(k, device=cuda) + 0.5
+    d = rt.dequantize(w).double()
+    _close(rt.decode_matvec(w, x), x.double() @ d.t())
+    base = torch.randn((nb, rows), device=cuda)
+    y = rt.decode_matvec(w, x, dst=base.clone(), residual=True, awq=awq)
+    _close(y, base.double() + (x * awq).double() @ d.t())
+
+
+@pytest.mark.parametrize("nb", [4, 7])
+@pytest.mark.parametrize("name", [t for t in TYPES if t != "q6_k"])
+@pytest.mark.parametrize("rows,k", [(4096, 3584), (4104, 3584), (8200, 3584), (8200, 5120), (12304, 2560)])
+def test_fused_batch_plans(cuda, name, rows, k, nb):
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    gate, up = _weight(name, rows, k, 1), _weight(name, rows, k, 2)
+    x = torch.randn((nb, k), device=cuda)
+    g, u = (x.double() @ rt.dequantize(w).double().t() for w in (gate, up))
+    _close(rt.ffn_gate_up_swiglu(gate, up, x), g / (1 + torch.exp(-g)) * u)
+
+
+@pytest.mark.parametrize("name", [t for t in TYPES if t != "q8_0"])
+@pytest.mark.parametrize("rows", [4104, 6144])
+def test_long_rows_split(cuda, name, rows):
+    """Three tiles and two K splits in rounds (k = 13312 = 52 chunks), every replay the same bits."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    k, nb = 13312, 5
+    w = _weight(name, rows, k, rows)
+    assert rt.gemv_kernel(w, nb, workspace=True)["workspace_bytes"] > 0
+    ws = rt.decode_matvec_workspace(w, nb, device=cuda)
+    x = torch.randn((nb, k), device=cuda)
+    y = rt.decode_matvec(w, x, workspace=ws)
+    _close(y, x.double() @ rt.dequantize(w).double().t())
+    for _ in range(3):
+        assert torch.equal(rt.decode_matvec(w, x, workspace=ws), y)
