@@ -76,6 +76,13 @@ hipError_t kq_gf4_swiglu(const GemvArgs& a, hipStream_t stream);
 namespace {
 
 
+// kStride, the LDS bytes of a transposed row, is 4, 12, 20 or 28 dwords mod 32:
+// the operand reads take 1 to 4 consecutive dwords of 16 rows per lane group,
+// and with an odd multiple of four dwords eight rows cover the banks once.
+// (With strides of 8, 16 or 24 mod 32 -- 16 bytes of pad behind 272, 144, 176
+// and 80 -- half of the LDS cycles were bank conflicts: Q6_K head b1 65.1 ->
+// 44.7 M LDS cycles, 179.3 -> 170.9 us; Q5_K 5120/17408 FFN b5 160.3 -> 156.1;
+// q8_0 12352x4096 b8 3.61 -> 2.20 M; 9B step b8 2005 -> 1969 us.)
 constexpr int kFmtQ8 = 0;
 constexpr int kFmtQ4K = 1;
 constexpr int kFmtGF4 = 2;
@@ -89,14 +96,14 @@ template <>
 struct Fmt<kFmtQ8> {
     static constexpr int kChunkBytes = 272;  // 8 blocks of 34 bytes = 256 columns
     static constexpr int kSegs = 17;         // 16-byte segments per row chunk
-    static constexpr int kStride = 288;      // LDS bytes per transposed row (16-byte pad)
+    static constexpr int kStride = 272;      // LDS bytes per transposed row
     static constexpr int kTypeId = 8;
 };
 template <>
 struct Fmt<kFmtQ4K> {
     static constexpr int kChunkBytes = 144;  // one super-block = 256 columns
     static constexpr int kSegs = 9;
-    static constexpr int kStride = 160;
+    static constexpr int kStride = 144;
     static constexpr int kTypeId = 12;
 };
 
@@ -111,24 +118,22 @@ template <>
 struct Fmt<kFmtQ5K> {
     static constexpr int kChunkBytes = 176;  // one super-block = 256 columns
     static constexpr int kSegs = 11;
-    static constexpr int kStride = 192;
+    static constexpr int kStride = 176;
     static constexpr int kTypeId = 13;
 };
 template <>
 struct Fmt<kFmtGF2> {
     static constexpr int kChunkBytes = 80;  // 16 code words + 16 scale bytes = 256 columns
     static constexpr int kSegs = 5;
-    static constexpr int kStride = 96;
+    static constexpr int kStride = 80;
     static constexpr int kTypeId = 101;
 };
 template <>
 struct Fmt<kFmtQ6K> {
     static constexpr int kChunkBytes = 210;  // one super-block = 256 columns
     static constexpr int kSegs = 14;         // aligned segments covering bytes [210c, 210c + 210)
-    // No pad (2-way bank conflicts on the transposed reads) so that two 16-wave
-    // workgroups fit a CU's LDS; the 2-byte realignment of d may read 4 bytes
-    // past a row, still inside the wave's block (the activation buffer follows).
-    static constexpr int kStride = 224;
+    // (one 16-byte segment of pad: 60 dwords)
+    static constexpr int kStride = 240;
     static constexpr int kTypeId = 14;
 };
 
