@@ -93,7 +93,7 @@ __global__ __launch_bounds__(kEncodeThreads) void gf4_pack_kernel(const float* _
 // flight per wave.  The encoders are bound by their fp32 reads and the IEEE
 // divides.  A thread per super-block (1 KB apart, three passes over its
 // columns) took 1061 us for Q4_K 12288x4096 with a column scale (0.22 TB/s);
-// this form takes 61 (3.8 TB/s; GF2 47, Q6_K 61).
+// this form takes 60.6 (3.8 TB/s; GF2 45, Q5_K 63, Q6_K 54).
 constexpr int kSuperUnroll = 4;
 constexpr int kEncodeWaves = kEncodeThreads / 64;
 
@@ -126,12 +126,16 @@ __device__ __forceinline__ float dpp_fmin(float v) {
 }
 
 // r[q] = rint(fl(n[q] / d) * mul + add) in the IEEE steps that the formats
-// state, without an IEEE divide where it cannot matter: t = n * rcp(d) is
-// within a few ulp of the quotient, so for |t| < 256 both round to the same
-// integer unless t lies within 0.001 of a tie; only a wave that holds such a
-// lane (or a divisor outside rcp's accurate range) divides.  d != 0.
+// state, without an IEEE divide where it cannot matter.  t = n * rcp(d) has a
+// relative error of at most 2^-22 against the rounded quotient (rcp within one
+// ulp, two roundings, the quotient's own), the affine form three more roundings
+// of 2^-24: below 2^-15 for |t| < 64, so both round to the same integer unless
+// t lies within 2^-14 of a tie.  Only a wave that holds such a lane (or a
+// divisor outside rcp's accurate range) divides: 3% of them with 256 codes
+// (a band of 0.001 and |t| < 256 sent 40% there).  d != 0.
 // (Q4_K 12288x4096 with a column scale: 87.5 -> 64.0 us with this and the
-// shared sub-block arithmetic of k_quantize_kernel.)
+// shared sub-block arithmetic of k_quantize_kernel; the narrower band 65.6 ->
+// 60.6, Q5_K 67.5 -> 63.0, GF2 47.7 -> 45.2)
 template <bool AFFINE>
 __device__ __forceinline__ void rint_div4(const float (&n)[4], float d, float (&r)[4]) {
     const float inv = __builtin_amdgcn_rcpf(d);
@@ -144,7 +148,7 @@ __device__ __forceinline__ void rint_div4(const float (&n)[4], float d, float (&
         far = fmaxf(far, fabsf(t - r[q]));
         big = fmaxf(big, fabsf(t));
     }
-    const bool sure = far < 0.499f && big < 256.0f && fabsf(d) > 0x1p-100f && fabsf(d) < 0x1p+100f;
+    const bool sure = far < 0.5f - 0x1p-14f && big < 64.0f && fabsf(d) > 0x1p-100f && fabsf(d) < 0x1p+100f;
     if (__any(!sure)) {
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
@@ -152,6 +156,14 @@ __device__ __forceinline__ void rint_div4(const float (&n)[4], float d, float (&
             r[q] = rintf(AFFINE ? __fadd_rn(__fmul_rn(t, 1.5f), 1.5f) : t);
         }
     }
+}
+
+// Four whole numbers in [0, 255] -> one per byte.
+__device__ __forceinline__ uint32_t pack_u8(const float (&r)[4]) {
+    uint32_t code = 0;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) code = __builtin_amdgcn_cvt_pk_u8_f32(r[q], q, code);
+    return code;
 }
 
 // GF2 super-blocks (256 columns = 16 groups of 16; this library's encoder, the
@@ -327,10 +339,9 @@ __global__ __launch_bounds__(kEncodeThreads) void k_quantize_kernel(const float*
 #pragma unroll
             for (int q = 0; q < 4; ++q) n[q] = __fadd_rn(v[u][q], offs);
             rint_div4<false>(n, step != 0.0f ? step : 1.0f, r);
-            uint32_t code = 0;  // the lane's four codes, one per byte
 #pragma unroll
-            for (int q = 0; q < 4; ++q)
-                code |= (step != 0.0f ? (uint32_t)fminf(fmaxf(r[q], 0.0f), kLevels) : 0u) << (8 * q);
+            for (int q = 0; q < 4; ++q) r[q] = fminf(fmaxf(r[q], 0.0f), kLevels);
+            const uint32_t code = step != 0.0f ? pack_u8(r) : 0u;  // the lane's four codes
             uint8_t* blk = dst + kBlockBytes * (i0 + u);  // 144- or 176-byte blocks: 16-byte aligned
             // nibbles: sub-blocks 2c and 2c + 1 are 8 lanes apart
             const uint32_t other = (uint32_t)__shfl_xor((int)code, 8);
@@ -369,7 +380,9 @@ __global__ __launch_bounds__(kEncodeThreads) void k_quantize_kernel(const float*
 // stored as ggml lays Q6_K out (qw35_types.metal:17-22): element
 // 128h + 32g + l has its low nibble in ql[64h + 32(g&1) + l] (high nibble for
 // g >= 2) and its top two bits at bit 2g of qh[32h + l].  Super-blocks are
-// 210 bytes (2-byte aligned), so a word leaves as two 16-bit stores.
+// 210 bytes (2-byte aligned), so a word leaves as two 16-bit stores.  With the
+// sub-block arithmetic per super-block instead of once for four, and the wider
+// band of rint_div4, 12288x4096 with a column scale took 72.6 us, now 54.2.
 __global__ __launch_bounds__(kEncodeThreads) void q6_k_quantize_kernel(const float* __restrict__ src,
                                                                        const float* __restrict__ col_scale,
                                                                        uint8_t* __restrict__ dst, uint64_t n_blocks,
@@ -383,29 +396,37 @@ __global__ __launch_bounds__(kEncodeThreads) void q6_k_quantize_kernel(const flo
     for (uint64_t i0 = wave * kSuperUnroll; i0 < n_blocks; i0 += (uint64_t)gridDim.x * kEncodeWaves * kSuperUnroll) {
         float v[kSuperUnroll][4];
         load_super(src, col_scale, i0, n_blocks, blocks_per_row, lane, v);
+        // lane l keeps the sub-block maximum of super-block l % 4, so the
+        // sub-block arithmetic (three divides) runs once for the four
+        static_assert(kSuperUnroll == 4, "one lane of a quad per super-block");
+        float amax_u = 0.0f;
+#pragma unroll
+        for (int u = 0; u < kSuperUnroll; ++u) {
+            float amax = fmaxf(fmaxf(fabsf(v[u][0]), fabsf(v[u][1])), fmaxf(fabsf(v[u][2]), fabsf(v[u][3])));
+            amax = dpp_fmax<kDppQuadXor2>(dpp_fmax<kDppQuadXor1>(amax));
+            amax_u = (lane & 3) == u ? amax : amax_u;
+        }
+        const float sub = __fdiv_rn(amax_u, 31.0f);
+        float smax = sub;
+#pragma unroll
+        for (int o = 4; o < 64; o <<= 1) smax = fmaxf(smax, __shfl_xor(smax, o));
+        const uint32_t d_bits_u = f32_to_f16_bits(__fdiv_rn(smax, 127.0f));
+        const float df = f16_bits_to_f32(d_bits_u);
+        const float a = (df != 0.0f) ? rintf(__fdiv_rn(sub, df)) : 0.0f;
+        const float scq = fminf(fmaxf(a, 0.0f), 127.0f);
+        const float step_u = __fmul_rn(df, scq);
+        const uint32_t sd_u = (uint32_t)(int)scq | (d_bits_u << 16);
 #pragma unroll
         for (int u = 0; u < kSuperUnroll; ++u) {
             if (i0 + u >= n_blocks) break;
-            float amax = fmaxf(fmaxf(fabsf(v[u][0]), fabsf(v[u][1])), fmaxf(fabsf(v[u][2]), fabsf(v[u][3])));
-            amax = dpp_fmax<kDppQuadXor1>(amax);
-            amax = dpp_fmax<kDppQuadXor2>(amax);
-            const float sub = __fdiv_rn(amax, 31.0f);
-            float smax = sub;
-#pragma unroll
-            for (int o = 4; o < 64; o <<= 1) smax = fmaxf(smax, __shfl_xor(smax, o));
-            const uint32_t d_bits = f32_to_f16_bits(__fdiv_rn(smax, 127.0f));
-            const float df = f16_bits_to_f32(d_bits);
-            const float a = (df != 0.0f) ? rintf(__fdiv_rn(sub, df)) : 0.0f;
-            const float scq = fminf(fmaxf(a, 0.0f), 127.0f);
-            const float step = __fmul_rn(df, scq);
+            const int from = (lane & ~3) | u;  // this sub-block's lane of super-block u
+            const float step = __shfl(step_u, from);
+            const uint32_t sd = (uint32_t)__shfl((int)sd_u, from);
             float r[4];
             rint_div4<false>(v[u], step != 0.0f ? step : 1.0f, r);
-            uint32_t code = 0;  // the lane's four codes, one per byte
 #pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const float qf = step != 0.0f ? r[q] : 0.0f;
-                code |= (uint32_t)(int)(fminf(fmaxf(qf, -32.0f), 31.0f) + 32.0f) << (8 * q);
-            }
+            for (int q = 0; q < 4; ++q) r[q] = fminf(fmaxf(r[q], -32.0f), 31.0f) + 32.0f;
+            const uint32_t code = step != 0.0f ? pack_u8(r) : 0x20202020u;  // the lane's four codes
             uint8_t* blk = dst + 210 * (i0 + u);
             // lane = 32h + 8g + l / 4: groups g and g + 2 share the bytes of ql, all four those of qh
             const int h = lane >> 5, g = (lane >> 3) & 3, l = 4 * (lane & 7);
@@ -415,8 +436,8 @@ __global__ __launch_bounds__(kEncodeThreads) void q6_k_quantize_kernel(const flo
             qh |= (uint32_t)__shfl_xor((int)qh, 16);
             if (g < 2) store4(blk + 64 * h + 32 * g + l, (code & 0x0F0F0F0Fu) | ((other & 0x0F0F0F0Fu) << 4));
             if (g == 2) store4(blk + 128 + 32 * h + l, qh);
-            if ((lane & 3) == 0) blk[192 + (lane >> 2)] = (uint8_t)(int)scq;
-            if (lane == 1) *reinterpret_cast<uint16_t*>(blk + 208) = (uint16_t)d_bits;
+            if ((lane & 3) == 0) blk[192 + (lane >> 2)] = (uint8_t)sd;
+            if (lane == 1) *reinterpret_cast<uint16_t*>(blk + 208) = (uint16_t)(sd >> 16);
         }
     }
 }
