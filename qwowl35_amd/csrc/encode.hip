@@ -90,10 +90,10 @@ __global__ __launch_bounds__(kEncodeThreads) void gf4_pack_kernel(const float* _
 // super-block, four consecutive columns per lane, so a super-block is one
 // coalesced 1 KB load, its group maxima are lane reductions and its packed
 // words one or two narrow stores; kSuperUnroll super-blocks' loads are in
-// flight per wave.  The encoders are bound by their fp32 reads and the IEEE
-// divides.  A thread per super-block (1 KB apart, three passes over its
+// flight per wave.  The encoders are bound by their fp32 reads and, for the
+// k-quants, VALU issue (the sub-blocks' arithmetic, the rounding of the codes).  A thread per super-block (1 KB apart, three passes over its
 // columns) took 1061 us for Q4_K 12288x4096 with a column scale (0.22 TB/s);
-// this form takes 60.6 (3.8 TB/s; GF2 45, Q5_K 63, Q6_K 54).
+// this form takes 52.5 (4.4 TB/s; GF2 45, Q5_K 54, Q6_K 53).
 constexpr int kSuperUnroll = 4;
 constexpr int kEncodeWaves = kEncodeThreads / 64;
 
@@ -107,13 +107,14 @@ __device__ __forceinline__ void load_super(const float* __restrict__ src, const 
     for (int u = 0; u < kSuperUnroll; ++u) {
         const uint64_t i = i0 + u < n_blocks ? i0 + u : n_blocks - 1;
         x[u] = *reinterpret_cast<const float4_t*>(src + 256 * i + 4 * lane);
+        s[u] = float4_t{1.0f, 1.0f, 1.0f, 1.0f};
         if (col_scale)
             s[u] = *reinterpret_cast<const float4_t*>(col_scale + 256u * mod_u64(i, blocks_per_row) + 4 * lane);
     }
 #pragma unroll
     for (int u = 0; u < kSuperUnroll; ++u)
 #pragma unroll
-        for (int q = 0; q < 4; ++q) v[u][q] = col_scale ? __fmul_rn(x[u][q], s[u][q]) : x[u][q];
+        for (int q = 0; q < 4; ++q) v[u][q] = __fmul_rn(x[u][q], s[u][q]);  // (a product needs no canonicalising max)
 }
 
 template <int CTRL>
@@ -125,31 +126,39 @@ __device__ __forceinline__ float dpp_fmin(float v) {
     return fminf(v, dpp_f32<CTRL>(v));
 }
 
+// 1 / d for rint_div4, or NaN where only the divide is sure to round right: a
+// quotient of n_max / d above 40 in magnitude or a divisor outside rcp's
+// accurate range.  n_max: the largest |n| that is divided by d.  d != 0.
+__device__ __forceinline__ float sure_rcp(float d, float n_max) {
+    const float inv = __builtin_amdgcn_rcpf(d);
+    const bool sure = n_max * fabsf(inv) < 40.0f && fabsf(d) > 0x1p-100f && fabsf(d) < 0x1p+100f;
+    return sure ? inv : __builtin_nanf("");
+}
+
 // r[q] = rint(fl(n[q] / d) * mul + add) in the IEEE steps that the formats
-// state, without an IEEE divide where it cannot matter.  t = n * rcp(d) has a
+// state, without an IEEE divide where it cannot matter.  t = n * inv has a
 // relative error of at most 2^-22 against the rounded quotient (rcp within one
 // ulp, two roundings, the quotient's own), the affine form three more roundings
 // of 2^-24: below 2^-15 for |t| < 64, so both round to the same integer unless
-// t lies within 2^-14 of a tie.  Only a wave that holds such a lane (or a
-// divisor outside rcp's accurate range) divides: 3% of them with 256 codes
-// (a band of 0.001 and |t| < 256 sent 40% there).  d != 0.
-// (Q4_K 12288x4096 with a column scale: 87.5 -> 64.0 us with this and the
-// shared sub-block arithmetic of k_quantize_kernel; the narrower band 65.6 ->
-// 60.6, Q5_K 67.5 -> 63.0, GF2 47.7 -> 45.2)
-template <bool AFFINE>
-__device__ __forceinline__ void rint_div4(const float (&n)[4], float d, float (&r)[4]) {
-    const float inv = __builtin_amdgcn_rcpf(d);
-    float far = 0.0f, big = 0.0f;
+// t lies within 2^-14 of a tie.  Only a wave that holds such a lane (or a NaN
+// inv) divides, by divisor(): 3% of them with 256 codes (a band of 0.001
+// sent 40% there).  (Q4_K 12288x4096 with a column scale: 87.5 -> 64.0 us with
+// this and the shared sub-block arithmetic of k_quantize_kernel; the narrower
+// band 65.6 -> 60.6, Q5_K 67.5 -> 63.0, GF2 47.7 -> 45.2)
+template <bool AFFINE, typename D>
+__device__ __forceinline__ void rint_div4(const float (&n)[4], float inv, D&& divisor, float (&r)[4]) {
+    float off[4];
 #pragma unroll
     for (int q = 0; q < 4; ++q) {
         float t = n[q] * inv;
         if (AFFINE) t = __builtin_fmaf(t, 1.5f, 1.5f);
         r[q] = rintf(t);
-        far = fmaxf(far, fabsf(t - r[q]));
-        big = fmaxf(big, fabsf(t));
+        off[q] = fabsf(t - r[q]);
     }
-    const bool sure = far < 0.5f - 0x1p-14f && big < 64.0f && fabsf(d) > 0x1p-100f && fabsf(d) < 0x1p+100f;
-    if (__any(!sure)) {
+    // (a NaN inv makes all four NaN, and fmaxf of NaNs is NaN)
+    const float far = fmaxf(fmaxf(off[0], off[1]), fmaxf(off[2], off[3]));
+    if (__any(!(far < 0.5f - 0x1p-14f))) {
+        const float d = divisor();
 #pragma unroll
         for (int q = 0; q < 4; ++q) {
             const float t = __fdiv_rn(n[q], d);
@@ -191,7 +200,8 @@ __global__ __launch_bounds__(kEncodeThreads) void gf2_pack_kernel(const float* _
             const uint32_t b = ((f32_to_f16_bits(amax) + 0x80u) >> 8) & 0xFFu;
             const float s = f16_bits_to_f32(b << 8);
             float r[4];
-            rint_div4<true>(v[u], s != 0.0f ? s : 1.0f, r);
+            const float div = s != 0.0f ? s : 1.0f;
+            rint_div4<true>(v[u], sure_rcp(div, amax), [&] { return div; }, r);
             uint32_t word = 0;
 #pragma unroll
             for (int q = 0; q < 4; ++q)  // s == 0: t = 0, code rint(1.5) = 2
@@ -329,20 +339,40 @@ __global__ __launch_bounds__(kEncodeThreads) void k_quantize_kernel(const float*
         const uint32_t mq_u = (uint32_t)fminf(fmaxf(m, 0.0f), 63.0f);
         const float step_u = __fmul_rn(df, (float)sc_u);
         const float offs_u = __fmul_rn(dminf, (float)mq_u);
-        const uint32_t both_u = sc_u | (mq_u << 8), dd_u = d_bits_u | (dmin_bits_u << 16);
+        const float div_u = step_u != 0.0f ? step_u : 1.0f;
+        const float inv_u = sure_rcp(div_u, fmaxf(fabsf(__fadd_rn(lo_u, offs_u)), fabsf(__fadd_rn(hi_u, offs_u))));
+        const unsigned long long zero = __ballot(step_u == 0.0f);
+        // headers: lane u of the first quad gathers those of super-block u
+        // (assembled per super-block, with its reciprocal and the largest
+        // quotient per lane: Q4_K 12288x4096 60.8 us, now 52.5; Q5_K 62.5 / 54.2).
+        // Sub-block j < 4 gives scale bytes j, j + 4 and j + 8, of its own
+        // scale and min and those of sub-block j + 4 (32 lanes on).
+        const uint32_t both = sc_u | (mq_u << 8);
+        const uint32_t upper = (uint32_t)__shfl_xor((int)both, 32);
+        const uint32_t s1 = upper & 63u, m1 = upper >> 8;
+        uint32_t w[3] = {(sc_u | ((s1 >> 4) << 6)) << (8 * (j & 3)), (mq_u | ((m1 >> 4) << 6)) << (8 * (j & 3)),
+                         ((s1 & 15u) | ((m1 & 15u) << 4)) << (8 * (j & 3))};
+#pragma unroll
+        for (int q = 0; q < 3; ++q) {
+            w[q] |= (uint32_t)__shfl_xor((int)w[q], 8);
+            w[q] |= (uint32_t)__shfl_xor((int)w[q], 16);
+        }
+        if (lane < kSuperUnroll && i0 + lane < n_blocks)  // 144- or 176-byte blocks: 16-byte aligned
+            *reinterpret_cast<uint4_t*>(dst + kBlockBytes * (i0 + lane)) =
+                uint4_t{d_bits_u | (dmin_bits_u << 16), w[0], w[1], w[2]};
 #pragma unroll
         for (int u = 0; u < kSuperUnroll; ++u) {
             if (i0 + u >= n_blocks) break;
             const int from = (lane & ~3) | u;  // this sub-block's lane of super-block u
-            const float step = __shfl(step_u, from), offs = __shfl(offs_u, from);
+            const float inv = __shfl(inv_u, from), offs = __shfl(offs_u, from);
             float n[4], r[4];
 #pragma unroll
             for (int q = 0; q < 4; ++q) n[q] = __fadd_rn(v[u][q], offs);
-            rint_div4<false>(n, step != 0.0f ? step : 1.0f, r);
+            rint_div4<false>(n, inv, [&] { return __shfl(div_u, from); }, r);
 #pragma unroll
             for (int q = 0; q < 4; ++q) r[q] = fminf(fmaxf(r[q], 0.0f), kLevels);
-            const uint32_t code = step != 0.0f ? pack_u8(r) : 0u;  // the lane's four codes
-            uint8_t* blk = dst + kBlockBytes * (i0 + u);  // 144- or 176-byte blocks: 16-byte aligned
+            const uint32_t code = (zero >> from) & 1 ? 0u : pack_u8(r);  // the lane's four codes
+            uint8_t* blk = dst + kBlockBytes * (i0 + u);
             // nibbles: sub-blocks 2c and 2c + 1 are 8 lanes apart
             const uint32_t other = (uint32_t)__shfl_xor((int)code, 8);
             if ((lane & 8) == 0)
@@ -354,21 +384,6 @@ __global__ __launch_bounds__(kEncodeThreads) void k_quantize_kernel(const float*
                 for (int o = 8; o < 64; o <<= 1) qh |= (uint32_t)__shfl_xor((int)qh, o);
                 if (lane < 8) reinterpret_cast<uint32_t*>(blk + 16)[lane] = qh;
             }
-            // header: lane q < 4 holds scale bytes q, q + 4 and q + 8
-            const uint32_t lo_j = (uint32_t)__shfl((int)both_u, 8 * (lane & 3) + u);
-            const uint32_t hi_j = (uint32_t)__shfl((int)both_u, 8 * (lane & 3) + 32 + u);
-            const uint32_t dd = (uint32_t)__shfl((int)dd_u, u);
-            const uint32_t s0 = lo_j & 63u, m0 = lo_j >> 8, s1 = hi_j & 63u, m1 = hi_j >> 8;
-            uint32_t w0 = (s0 | ((s1 >> 4) << 6)) << (8 * (lane & 3));
-            uint32_t w1 = (m0 | ((m1 >> 4) << 6)) << (8 * (lane & 3));
-            uint32_t w2 = ((s1 & 15u) | ((m1 & 15u) << 4)) << (8 * (lane & 3));
-            w0 |= dpp_u32<kDppQuadXor1>(w0);
-            w1 |= dpp_u32<kDppQuadXor1>(w1);
-            w2 |= dpp_u32<kDppQuadXor1>(w2);
-            w0 |= dpp_u32<kDppQuadXor2>(w0);
-            w1 |= dpp_u32<kDppQuadXor2>(w1);
-            w2 |= dpp_u32<kDppQuadXor2>(w2);
-            if (lane == 0) *reinterpret_cast<uint4_t*>(blk) = uint4_t{dd, w0, w1, w2};
         }
     }
 }
@@ -382,7 +397,7 @@ __global__ __launch_bounds__(kEncodeThreads) void k_quantize_kernel(const float*
 // g >= 2) and its top two bits at bit 2g of qh[32h + l].  Super-blocks are
 // 210 bytes (2-byte aligned), so a word leaves as two 16-bit stores.  With the
 // sub-block arithmetic per super-block instead of once for four, and the wider
-// band of rint_div4, 12288x4096 with a column scale took 72.6 us, now 54.2.
+// band of rint_div4, 12288x4096 with a column scale took 72.6 us, now 53.1.
 __global__ __launch_bounds__(kEncodeThreads) void q6_k_quantize_kernel(const float* __restrict__ src,
                                                                        const float* __restrict__ col_scale,
                                                                        uint8_t* __restrict__ dst, uint64_t n_blocks,
@@ -415,18 +430,21 @@ __global__ __launch_bounds__(kEncodeThreads) void q6_k_quantize_kernel(const flo
         const float a = (df != 0.0f) ? rintf(__fdiv_rn(sub, df)) : 0.0f;
         const float scq = fminf(fmaxf(a, 0.0f), 127.0f);
         const float step_u = __fmul_rn(df, scq);
-        const uint32_t sd_u = (uint32_t)(int)scq | (d_bits_u << 16);
+        const float div_u = step_u != 0.0f ? step_u : 1.0f;
+        const float inv_u = sure_rcp(div_u, amax_u);
+        // scale and fp16 scale of the super-block; bit 8: all codes are zero
+        const uint32_t sd_u = (uint32_t)(int)scq | (step_u == 0.0f ? 256u : 0u) | (d_bits_u << 16);
 #pragma unroll
         for (int u = 0; u < kSuperUnroll; ++u) {
             if (i0 + u >= n_blocks) break;
             const int from = (lane & ~3) | u;  // this sub-block's lane of super-block u
-            const float step = __shfl(step_u, from);
+            const float inv = __shfl(inv_u, from);
             const uint32_t sd = (uint32_t)__shfl((int)sd_u, from);
             float r[4];
-            rint_div4<false>(v[u], step != 0.0f ? step : 1.0f, r);
+            rint_div4<false>(v[u], inv, [&] { return __shfl(div_u, from); }, r);
 #pragma unroll
             for (int q = 0; q < 4; ++q) r[q] = fminf(fmaxf(r[q], -32.0f), 31.0f) + 32.0f;
-            const uint32_t code = step != 0.0f ? pack_u8(r) : 0x20202020u;  // the lane's four codes
+            const uint32_t code = (sd & 256u) ? 0x20202020u : pack_u8(r);  // the lane's four codes
             uint8_t* blk = dst + 210 * (i0 + u);
             // lane = 32h + 8g + l / 4: groups g and g + 2 share the bytes of ql, all four those of qh
             const int h = lane >> 5, g = (lane >> 3) & 3, l = 4 * (lane & 7);

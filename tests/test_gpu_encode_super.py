@@ -36,3 +36,29 @@ def test_super_block_encoders_bit_exact(cuda, name, rows, k, scaled):
     v = (w * s[None, :]).astype(np.float32) if scaled else w
     want = oq6.q6_k_quantize(v) if name == "q6_k" else om.quantize(CODECS[name], v)
     assert np.array_equal(got.cpu().numpy().reshape(rows, -1), np.asarray(want).reshape(rows, -1).view(np.uint8))
+
+
+@pytest.mark.parametrize("name", ["q4_k", "q5_k", "q6_k"])
+def test_sub_blocks_far_below_the_largest(cuda, name):
+    """Sub-blocks whose range is just under 1.5 steps of the super-block's scale,
+    so that scale code 1 leaves quotients far past the last code, beside ranges
+    that round to scale code 0 and one that is zero throughout."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    rng = np.random.default_rng(7)
+    rows, k = 8, 512
+    steps = 127.0 if name == "q6_k" else 63.0
+    w = rng.uniform(-1.0, 1.0, (rows, k)).astype(np.float32)
+    w[:, ::16] = 1.0
+    w[:, 1::16] = -1.0  # every 16- and 32-column range the same
+    ratio = np.ones((rows, k), dtype=np.float32)
+    ratio[:, 32:96] = 1.48 / steps
+    ratio[:, 96:128] = 0.4 / steps
+    ratio[:, 128:160] = 0.0
+    ratio[:, 288:512] = 1.47 / steps
+    v = w * ratio * np.float32(0.7)
+    got = rt.quantize(torch.from_numpy(v).to(cuda), CODECS[name]).cpu().numpy().reshape(rows, -1)
+    want = oq6.q6_k_quantize(v) if name == "q6_k" else om.quantize(CODECS[name], v)
+    assert np.array_equal(got, np.asarray(want).reshape(rows, -1).view(np.uint8))
