@@ -251,11 +251,14 @@ def load(path: str | os.PathLike | None = None) -> C.CDLL:
     return lib
 
 
+_ErrBuffer = C.c_char * 512
+
+
 def call(name: str, *args) -> int:
     """Call ``name(*args, err, err_len)`` and raise ``Qw35Error`` on a 0 / NULL return."""
     lib = load()
-    err = C.create_string_buffer(512)
-    rc = getattr(lib, name)(*args, err, C.sizeof(err))
+    err = _ErrBuffer()
+    rc = getattr(lib, name)(*args, err, 512)
     if not rc:
         raise Qw35Error(f"{name}: {err.value.decode(errors='replace')}")
     return rc

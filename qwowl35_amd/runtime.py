@@ -207,8 +207,8 @@ def _ptr(t: torch.Tensor | None) -> C.c_void_p:
 
 
 def _stream(stream) -> C.c_void_p:
-    if stream is None:
-        stream = torch.cuda.current_stream()
+    if stream is None:  # the current stream's handle, without a torch.cuda.Stream object for each call
+        return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
     return C.c_void_p(stream.cuda_stream)
 
 
