@@ -86,14 +86,15 @@ __global__ __launch_bounds__(kEncodeThreads) void gf4_pack_kernel(const float* _
     }
 }
 
-// Super-block encoders (GF2, Q4_K, Q5_K, Q6_K; q8_0 likewise): one wave per 256-column
-// super-block, four consecutive columns per lane, so a super-block is one
-// coalesced 1 KB load, its group maxima are lane reductions and its packed
-// words one or two narrow stores; kSuperUnroll super-blocks' loads are in
-// flight per wave.  The encoders are bound by their fp32 reads and, for the
-// k-quants, VALU issue (the sub-blocks' arithmetic, the rounding of the codes).  A thread per super-block (1 KB apart, three passes over its
-// columns) took 1061 us for Q4_K 12288x4096 with a column scale (0.22 TB/s);
-// this form takes 52.5 (4.4 TB/s; GF2 45, Q5_K 54, Q6_K 53).
+// Super-block encoders (GF2, Q4_K, Q5_K, Q6_K; q8_0 likewise): one wave per
+// 256-column super-block, four consecutive columns per lane, so a super-block
+// is one coalesced 1 KB load, its group maxima are lane reductions and its
+// packed words one or two narrow stores; kSuperUnroll super-blocks' loads are
+// in flight per wave.  The encoders are bound by their fp32 reads and, for the
+// k-quants, VALU issue (the sub-blocks' arithmetic, the rounding of the codes).
+// A thread per super-block (1 KB apart, three passes over its columns) took
+// 1061 us for Q4_K 12288x4096 with a column scale (0.22 TB/s); this form takes
+// 52.5 (4.4 TB/s; GF2 45, Q5_K 54, Q6_K 53).
 constexpr int kSuperUnroll = 4;
 constexpr int kEncodeWaves = kEncodeThreads / 64;
 
