@@ -980,6 +980,10 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
             return {3, 8, 2, 1};
         }
         if (swiglu) return {2, 12, 2, 1};
+        // q8_0 rows of up to 2048 columns at batch 3..4: one tile, all of a
+        // row's chunks at once (greedy head 151936x2048 b3 80.7 us, with four
+        // tiles 111.4; 32000x2048 22.2 / 28.6; at batch 8 208 against 128)
+        if (fmt == kFmtQ8 && nb < 8 && chunks <= 8) return {1, 8, 1, 1};
         return {4, 8, 2, 1};
     }
     // Longer rows: eight waves of four chunks per round (kq_mfma_gemv_long).
