@@ -1096,14 +1096,15 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
         total_rows = 0;
         for (int s = 0; s < a.n_seg; ++s) total_rows += a.seg_rows[s];
     }
-    KqPlan p = plan_kq(FMT, total_rows, a.k, NB, a.ks_ws != nullptr && !a.am_token, SWIGLU);
+    // (the fused form has no split: its plans come without one, also in a recorded step, which has a workspace)
+    KqPlan p = plan_kq(FMT, total_rows, a.k, NB, a.ks_ws != nullptr && !a.am_token && !SWIGLU, SWIGLU);
     if (p.s > 1) {
         int groups = (a.rows + 16 * p.rt - 1) / (16 * p.rt);
         if (a.n_seg > 1) {
             groups = 0;
             for (int s = 0; s < a.n_seg; ++s) groups += (a.seg_rows[s] + 16 * p.rt - 1) / (16 * p.rt);
         }
-        if (groups > kKsCounters || a.ks_ws_bytes < kq_split_ws_bytes(groups, p.s, p.rt, NB, SWIGLU ? 2 : 1))
+        if (groups > kKsCounters || a.ks_ws_bytes < kq_split_ws_bytes(groups, p.s, p.rt, NB, 1))
             p = plan_kq(FMT, total_rows, a.k, NB, false, SWIGLU);
     }
 #define QW35_KQ_PLAN(RT, KS, CPW, P)                                                             \

@@ -86,3 +86,22 @@ def test_long_rows_split(cuda, name, rows):
     _close(y, x.double() @ rt.dequantize(w).double().t())
     for _ in range(3):
         assert torch.equal(rt.decode_matvec(w, x, workspace=ws), y)
+
+
+@pytest.mark.parametrize("name", [t for t in TYPES if t != "q6_k"])
+@pytest.mark.parametrize("rows,k", [(4104, 13312), (1000, 12288)])
+def test_recorded_fused_long_rows(cuda, name, rows, k):
+    """A recorded gate/up op of a shape whose plain GEMV splits K (recorded ops have a workspace)."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    nb = 5
+    gate, up = _weight(name, rows, k, 1), _weight(name, rows, k, 2)
+    x, y = torch.randn((nb, k), device=cuda), torch.empty((nb, rows), device=cuda)
+    plan = rt.DecodePlan()
+    plan.swiglu(gate, up, x, y)
+    plan.record()
+    plan.launch()
+    rt.sync()
+    assert torch.equal(y, rt.ffn_gate_up_swiglu(gate, up, x))

@@ -1,0 +1,37 @@
+"""Every shape that the GEMV entry points accept names a launch.
+
+The launch planner picks a kernel by codec, batch, row tiles and 256-column
+chunks; a plan without an instantiation is an error of the call (and of
+recording a decode plan, whose ops are described with a K-split workspace).
+qw35_hip_gemv_kernel describes the launch without a GPU, so this walks both
+sides of every bound of the planner: plain and fused, with and without a
+workspace."""
+from __future__ import annotations
+
+import pytest
+
+from qwowl35_amd import _ffi
+from tests.test_plan_coverage import GF2, GF4, Q4K, Q5K, Q6K, Q8, kernel
+
+# row tiles of 16 on both sides of 256, 384, 512, 768, 1280 and 4096, ragged last tiles among them
+ROWS = [16, 1000, 4096, 4104, 6144, 6152, 8192, 8200, 12288, 12296, 17408, 20488, 65536, 65552]
+CHUNKS = [1, 2, 4, 6, 8, 10, 12, 14, 16, 18, 24, 26, 32, 34, 48, 50, 52, 64, 68, 96, 98, 256]
+
+
+@pytest.fixture(scope="module")
+def lib():
+    return _ffi.load()
+
+
+@pytest.mark.parametrize("type_id", [GF4, GF2, Q8, Q4K, Q5K, Q6K])
+@pytest.mark.parametrize("ws", [False, True])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_every_shape_has_a_launch(lib, type_id, swiglu, ws):
+    if swiglu and type_id == Q6K:
+        pytest.skip("no fused q6_k")
+    for rows in ROWS:
+        for chunks in CHUNKS:  # (even counts: q6_k takes k % 512 == 0)
+            if type_id == Q6K and chunks % 2:
+                continue
+            for nb in range(1, 9):
+                assert kernel(type_id, rows, 256 * chunks, nb, swiglu=swiglu, ws=ws), (rows, chunks, nb)
