@@ -202,7 +202,10 @@ int qw35_hip_gemv_kernel(const qw35_hip_weight *w, const qw35_hip_weight *w_up, 
  * reference's head is Q6_K or GF4).  For the k-quants and GF2 the logits are
  * bit-identical to qw35_hip_decode_matvec's.  Two launches on `stream`;
  * workspace: device memory of qw35_hip_output_argmax_workspace_size(w, n_batch)
- * bytes (256-byte aligned, caller-owned, not shared by concurrent calls). */
+ * bytes (256-byte aligned, caller-owned, not shared by concurrent calls), which
+ * also serves every smaller batch; for heads of 65521 rows or more and
+ * 2304..4096 columns the size is that of n_batch alone, so a buffer for several
+ * batches takes the largest of their sizes. */
 uint64_t qw35_hip_output_argmax_workspace_size(const qw35_hip_weight *w, uint32_t n_batch);
 int qw35_hip_output_argmax(const qw35_hip_weight *w, const float *x, const float *awq, uint32_t n_batch,
                            uint32_t *token, float *logit, void *workspace, uint64_t workspace_bytes, void *stream,

@@ -299,6 +299,21 @@ uint64_t argmax_ws_part(const qw35_hip_weight* w, uint32_t n_batch) {
     return (n * 4 + 255) / 256 * 256;
 }
 
+// The size a caller is told: it holds the partials of every batch up to
+// n_batch, since a smaller batch's plan may have fewer row tiles per workgroup
+// and more partials (q8_0 151936 x 2048: 4 rows take 304128 bytes, 8 rows
+// 152064).  Vocabulary-sized heads keep the size of n_batch alone, the one
+// callers of that head have been told for each batch.
+uint64_t argmax_ws_bytes(const qw35_hip_weight* w, uint32_t n_batch) {
+    uint64_t part = argmax_ws_part(w, n_batch);
+    if (!qw35::argmax_head_sized((int)w->rows, (int)w->k))
+        for (uint32_t b = 1; b < n_batch; ++b) {
+            const uint64_t p = argmax_ws_part(w, b);
+            part = p > part ? p : part;
+        }
+    return 2 * part;
+}
+
 // A recorded decode-step plan: the launches (their weight pointers, shapes and
 // buffers baked into the kernel arguments) held as an instantiated hipGraph.
 struct Plan {
@@ -852,7 +867,7 @@ uint64_t qw35_hip_output_argmax_workspace_size(const qw35_hip_weight* w, uint32_
     if (!check_weight(w, "output_argmax", msg, sizeof msg) || !check_chunked_k(w, "", msg, sizeof msg) ||
         w->type_id == qw35::kTypeF16 || n_batch < 1 || n_batch > QW35_HIP_MAX_BATCH)
         return 0;
-    return 2 * argmax_ws_part(w, n_batch);
+    return argmax_ws_bytes(w, n_batch);
 }
 
 int qw35_hip_output_argmax(const qw35_hip_weight* w, const float* x, const float* awq, uint32_t n_batch,

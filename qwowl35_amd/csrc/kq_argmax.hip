@@ -66,6 +66,8 @@ int argmax_groups(uint32_t type_id, int rows, int k, int n_batch) {
     return (rows + 16 * p.rt - 1) / (16 * p.rt);
 }
 
+bool argmax_head_sized(int rows, int k) { return kq_head_sized(rows, k); }
+
 hipError_t launch_argmax_gemv(uint32_t type_id, const GemvArgs& a, uint32_t* token, float* logit,
                               hipStream_t stream) {
     if (!a.am_token || !a.am_logit || a.w_up || a.n_seg > 1) return hipErrorInvalidValue;

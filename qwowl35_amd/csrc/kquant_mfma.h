@@ -908,6 +908,9 @@ __global__ __launch_bounds__(64 * KS) void kq_mfma_gemv_long(GemvArgs args) {
     kq_gemv_body<FMT, NB, RT, KS, CPW, P, SWIGLU, HAS_AWQ, true>(args);
 }
 
+// Vocabulary-sized heads of 2304..4096 columns, whose plans are the codecs' own.
+inline bool kq_head_sized(int rows, int k) { return (rows + 15) / 16 >= 4096 && (k >> 8) > 8 && (k >> 8) <= 16; }
+
 struct KqPlan {
     int rt, ks, cpw, p;
     int s = 1;  // K splits across workgroups (needs a workspace)
@@ -941,8 +944,8 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
         if (split_ok && fmt != kFmtQ8 && tiles > 256 && tiles <= 384 && chunks > 48 && chunks % 2 == 0)
             return {3, 12, 2, 1, 2};
         if (chunks <= 4) return {1, 4, 1, 1};
-        if (tiles >= 4096 && chunks > 8 && chunks <= 16 && !swiglu) {
-            // LM-head sized: at batch 8 four tiles per 4-wave workgroup (head b8
+        if (kq_head_sized(rows, k) && !swiglu) {
+            // at batch 8 four tiles per 4-wave workgroup (head b8
             // Q4_K 199 us, Q6_K 278, Q5_K 249, GF2 176; with {2, 4, 4, 2} 234 /
             // 322 / 261 / 210 us); Q4_K eight tiles (one sweep on one box: 170.3
             // us against 173.5 with four, 175.9 with six; Q6_K 258.7 with eight,

@@ -81,6 +81,8 @@ hipError_t launch_q6_k_gemv(const GemvArgs& a, hipStream_t stream);
 // Greedy head: workgroups of the GEMV launch that launch_argmax_gemv makes for
 // (type_id, rows, k, n_batch) -- the number of partials per batch row.
 int argmax_groups(uint32_t type_id, int rows, int k, int n_batch);
+// Whether the head has the launch plans of a vocabulary-sized one.
+bool argmax_head_sized(int rows, int k);
 // GEMV with the argmax epilogue (a.am_token / a.am_logit hold
 // argmax_groups(...) * n_batch partials), then the reduction of the partials to
 // token[b], logit[b].

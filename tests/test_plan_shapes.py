@@ -8,10 +8,12 @@ sides of every bound of the planner: plain and fused, with and without a
 workspace."""
 from __future__ import annotations
 
+import ctypes as C
+
 import pytest
 
 from qwowl35_amd import _ffi
-from tests.test_plan_coverage import GF2, GF4, Q4K, Q5K, Q6K, Q8, kernel
+from tests.test_plan_coverage import GF2, GF4, Q4K, Q5K, Q6K, Q8, ROW_BYTES, kernel
 
 # row tiles of 16 on both sides of 256, 384, 512, 768, 1280 and 4096, ragged last tiles among them
 ROWS = [16, 1000, 4096, 4104, 6144, 6152, 8192, 8200, 12288, 12296, 17408, 20488, 65536, 65552]
@@ -35,3 +37,23 @@ def test_every_shape_has_a_launch(lib, type_id, swiglu, ws):
                 continue
             for nb in range(1, 9):
                 assert kernel(type_id, rows, 256 * chunks, nb, swiglu=swiglu, ws=ws), (rows, chunks, nb)
+
+
+@pytest.mark.parametrize("type_id", [GF4, GF2, Q8, Q4K, Q5K, Q6K])
+@pytest.mark.parametrize("rows,k", [(151936, 1024), (151936, 2048), (32000, 2048), (32000, 4096), (65552, 2048),
+                                    (20488, 2560), (151936, 5120), (100000, 6144)])
+def test_head_workspace_serves_smaller_batches(lib, type_id, rows, k):
+    """A workspace sized for some batch is accepted by calls of every smaller
+    one (the size is what the call asks for or more, and never falls)."""
+    w = _ffi.Weight()
+    w.data, w.k, w.rows, w.type_id, w.bytes = 256, k, rows, type_id, ROW_BYTES[type_id](k) * rows
+    sizes = [lib.qw35_hip_output_argmax_workspace_size(C.byref(w), nb) for nb in range(1, 9)]
+    assert sizes[0] > 0 and sizes == sorted(sizes), sizes
+    # what a call of each batch needs: its token and logit partials, one per workgroup and batch row
+    g = C.c_uint32()
+    for nb in range(1, 9):
+        if type_id == GF4:  # (the GF4 GEMV is another kernel than its head; covered by the sizes)
+            break
+        _ffi.call("qw35_hip_gemv_kernel", C.byref(w), None, nb, 0, 0, None, 0, C.byref(g), None, None, None)
+        need = 2 * ((4 * nb * g.value + 255) // 256 * 256)
+        assert all(size >= need for size in sizes[nb - 1:]), (nb, need, sizes)
