@@ -944,6 +944,20 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
         if (split_ok && fmt != kFmtQ8 && tiles > 256 && tiles <= 384 && chunks > 48 && chunks % 2 == 0)
             return {3, 12, 2, 1, 2};
         if (chunks <= 4) return {1, 4, 1, 1};
+        if (chunks <= 8) {
+            // All of a row's chunks at once, one per wave: a second chunk per
+            // wave is never live, but the workgroup still loads it (chunk 0
+            // again) and waits for it (us, one chunk per wave against two:
+            // fused Q4_K 16384x2048 b8 14.3 / 19.8, b3 13.0 / 16.9; q8_0
+            // 151936x2048 b8 100 / 117, 7168x2048 b3 7.2 / 7.6).
+            if (tiles <= 256) return {1, 8, 1, 1};
+            if (tiles <= 512) return {2, 8, 1, 1};
+            if (tiles <= 768) return swiglu && fmt == kFmtQ8 && nb < 8 ? KqPlan{1, 8, 1, 1} : KqPlan{3, 8, 1, 1};
+            if (swiglu) return {2, 8, 1, 1};
+            // q8_0 at batch 3..4: one tile (greedy head 151936x2048 b3 80.7 us,
+            // with four tiles 111.4 in two chunks per wave; 32000x2048 22.2 / 28.6)
+            return fmt == kFmtQ8 && nb < 8 ? KqPlan{1, 8, 1, 1} : KqPlan{4, 8, 1, 1};
+        }
         if (kq_head_sized(rows, k) && !swiglu) {
             // at batch 8 four tiles per 4-wave workgroup (head b8
             // Q4_K 199 us, Q6_K 278, Q5_K 249, GF2 176; with {2, 4, 4, 2} 234 /
@@ -968,9 +982,8 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
         // q8_0 9.2 -> 8.6 us, 8192x4096 11.9 -> 11.5), longer rows on twelve
         // waves in rounds; more tiles hold eight waves' loads.
         if (tiles <= 256)
-            return chunks <= 8 ? KqPlan{1, 8, 1, 1} : chunks > 12 && chunks <= 16 ? KqPlan{1, 16, 1, 1} : KqPlan{1, 12, 2, 1};
+            return chunks > 12 && chunks <= 16 ? KqPlan{1, 16, 1, 1} : KqPlan{1, 12, 2, 1};
         if (tiles <= 512) {
-            if (chunks <= 8) return {2, 8, 2, 1};
             // (two fused tiles per wave spill at sixteen waves)
             return chunks > 12 && chunks <= 16 && !swiglu ? KqPlan{2, 16, 1, 1} : KqPlan{2, 12, 2, 1};
         }
@@ -983,10 +996,6 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
             return {3, 8, 2, 1};
         }
         if (swiglu) return {2, 12, 2, 1};
-        // q8_0 rows of up to 2048 columns at batch 3..4: one tile, all of a
-        // row's chunks at once (greedy head 151936x2048 b3 80.7 us, with four
-        // tiles 111.4; 32000x2048 22.2 / 28.6; at batch 8 208 against 128)
-        if (fmt == kFmtQ8 && nb < 8 && chunks <= 8) return {1, 8, 1, 1};
         return {4, 8, 2, 1};
     }
     // Longer rows: eight waves of four chunks per round (kq_mfma_gemv_long).
@@ -1128,7 +1137,8 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
         QW35_KQ_PLAN(1, 8, 1, 1)
         QW35_KQ_PLAN(1, 16, 1, 1)
         QW35_KQ_ROUNDS(1, 12, 2, 1)
-        QW35_KQ_PLAN(2, 8, 2, 1)
+        QW35_KQ_PLAN(2, 8, 1, 1)
+        QW35_KQ_PLAN(3, 8, 1, 1)
         QW35_KQ_ROUNDS(2, 12, 2, 1)
         if constexpr (SWIGLU && FMT == kFmtQ8) {
             QW35_KQ_PLAN(3, 8, 2, 1)
@@ -1138,6 +1148,7 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
         }
         if constexpr (!SWIGLU) {
             QW35_KQ_PLAN(2, 16, 1, 1)
+            QW35_KQ_PLAN(4, 8, 1, 1)
             QW35_KQ_ROUNDS(4, 8, 2, 1)
             QW35_KQ_PLAN(4, 12, 1, 1)    // the K-split plans
             QW35_KQ_ROUNDS(3, 12, 2, 1)

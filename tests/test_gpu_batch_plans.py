@@ -105,3 +105,26 @@ def test_recorded_fused_long_rows(cuda, name, rows, k):
     plan.launch()
     rt.sync()
     assert torch.equal(y, rt.ffn_gate_up_swiglu(gate, up, x))
+
+
+@pytest.mark.parametrize("nb", [3, 8])
+@pytest.mark.parametrize("name", list(TYPES))
+@pytest.mark.parametrize("rows,k", [(4096, 2048), (4104, 1536), (8200, 2048), (12304, 1536)])
+def test_short_rows(cuda, name, rows, k, nb):
+    """Rows of at most eight chunks (one per wave): the fused form, and the greedy
+    head with a workspace that was sized for batch 8."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    w = _weight(name, rows, k, 1)
+    x = torch.randn((nb, k), device=cuda)
+    want = x.double() @ rt.dequantize(w).double().t()
+    if name != "q6_k":
+        up = _weight(name, rows, k, 2)
+        u = x.double() @ rt.dequantize(up).double().t()
+        _close(rt.ffn_gate_up_swiglu(w, up, x), want / (1 + torch.exp(-want)) * u)
+    token, logit = rt.output_argmax(w, x, workspace=rt.output_argmax_workspace(w, 8))
+    best = want.max(dim=1)
+    assert torch.equal(token.long(), best.indices)  # (random rows: no ties within 2e-6)
+    assert float((logit.double() - best.values).abs().max()) <= 2e-6 * float(want.norm(dim=1).max())

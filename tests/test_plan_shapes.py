@@ -57,3 +57,18 @@ def test_head_workspace_serves_smaller_batches(lib, type_id, rows, k):
         _ffi.call("qw35_hip_gemv_kernel", C.byref(w), None, nb, 0, 0, None, 0, C.byref(g), None, None, None)
         need = 2 * ((4 * nb * g.value + 255) // 256 * 256)
         assert all(size >= need for size in sizes[nb - 1:]), (nb, need, sizes)
+
+
+@pytest.mark.parametrize("type_id", [GF4, GF2, Q8, Q4K, Q5K, Q6K])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_short_rows_load_no_dead_chunk(lib, type_id, swiglu):
+    """Batch 3..8, rows of up to 2048 columns: no wave loads a chunk past the row."""
+    if swiglu and type_id == Q6K:
+        pytest.skip("no fused q6_k")
+    for rows in ROWS:
+        for chunks in (2, 4, 6, 8):
+            for nb in range(3, 9):
+                name = kernel(type_id, rows, 256 * chunks, nb, swiglu=swiglu)
+                if name.startswith("kq_"):  # <codec, batch, row tiles, waves, chunks per wave, ...>
+                    waves, per_wave = (int(v) for v in name.split("<")[1].split(",")[3:5])
+                    assert (per_wave - 1) * waves < chunks, (rows, chunks, nb, name)
