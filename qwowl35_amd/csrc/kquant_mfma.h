@@ -983,6 +983,16 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
         // waves in rounds; more tiles hold eight waves' loads.
         if (tiles <= 256)
             return chunks > 12 && chunks <= 16 ? KqPlan{1, 16, 1, 1} : KqPlan{1, 12, 2, 1};
+        // Fused q8_0, Q4_K and Q5_K of more than 24 chunks: two tiles in rounds
+        // need more registers than twelve waves leave (168 per lane; 96..104 of
+        // q8_0's spilled, 12..18 of the others'), so eight waves (us at b8,
+        // twelve / eight: 6144x8192 q8_0 85.8 / 33.6, Q4_K 30.2 / 25.1, Q5_K
+        // 34.2 / 28.2; GF4 and GF2 fit twelve).  q8_0 of more than two tiles
+        // per CU: one (12288x7168 b3 two on twelve waves 150, two on eight 52.6,
+        // one 42.9).
+        if (swiglu && chunks > 24 && tiles > 256 && fmt != kFmtGF4 && fmt != kFmtGF2 &&
+            (tiles <= 512 || tiles > 768 || fmt == kFmtQ8))
+            return fmt == kFmtQ8 && tiles > 512 ? KqPlan{1, 8, 2, 1} : KqPlan{2, 8, 2, 1};
         if (tiles <= 512) {
             // (two fused tiles per wave spill at sixteen waves)
             return chunks > 12 && chunks <= 16 && !swiglu ? KqPlan{2, 16, 1, 1} : KqPlan{2, 12, 2, 1};
@@ -1139,10 +1149,15 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
         QW35_KQ_ROUNDS(1, 12, 2, 1)
         QW35_KQ_PLAN(2, 8, 1, 1)
         QW35_KQ_PLAN(3, 8, 1, 1)
-        QW35_KQ_ROUNDS(2, 12, 2, 1)
+        if constexpr (SWIGLU && FMT != kFmtGF4 && FMT != kFmtGF2) {
+            QW35_KQ_PLAN(2, 12, 2, 1)
+            QW35_KQ_ROUNDS(2, 8, 2, 1)
+        } else {
+            QW35_KQ_ROUNDS(2, 12, 2, 1)
+        }
         if constexpr (SWIGLU && FMT == kFmtQ8) {
             QW35_KQ_PLAN(3, 8, 2, 1)
-            if constexpr (NB == 4) { QW35_KQ_PLAN(1, 8, 2, 1) }
+            QW35_KQ_ROUNDS(1, 8, 2, 1)
         } else {
             QW35_KQ_ROUNDS(3, 8, 2, 1)
         }
@@ -1151,7 +1166,7 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
             QW35_KQ_PLAN(4, 8, 1, 1)
             QW35_KQ_ROUNDS(4, 8, 2, 1)
             QW35_KQ_PLAN(4, 12, 1, 1)    // the K-split plans
-            QW35_KQ_ROUNDS(3, 12, 2, 1)
+            if constexpr (FMT != kFmtQ8) { QW35_KQ_ROUNDS(3, 12, 2, 1) }
             if constexpr (FMT == kFmtQ4K && NB == 8) { QW35_KQ_PLAN(8, 4, 4, 1) }
             if constexpr (FMT != kFmtQ8 && FMT != kFmtGF4) {
                 if constexpr (NB == 8) {

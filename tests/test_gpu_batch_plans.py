@@ -128,3 +128,18 @@ def test_short_rows(cuda, name, rows, k, nb):
     best = want.max(dim=1)
     assert torch.equal(token.long(), best.indices)  # (random rows: no ties within 2e-6)
     assert float((logit.double() - best.values).abs().max()) <= 2e-6 * float(want.norm(dim=1).max())
+
+
+@pytest.mark.parametrize("nb", [3, 8])
+@pytest.mark.parametrize("name", ["q8_0", "q4_k", "q5_k"])
+@pytest.mark.parametrize("rows,k", [(4104, 6400), (8200, 6400), (12304, 7168)])
+def test_fused_rounds(cuda, name, rows, k, nb):
+    """Fused rows of more than 24 chunks: eight waves in rounds, the last one partly idle."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    gate, up = _weight(name, rows, k, 1), _weight(name, rows, k, 2)
+    x = torch.randn((nb, k), device=cuda)
+    g, u = (x.double() @ rt.dequantize(w).double().t() for w in (gate, up))
+    _close(rt.ffn_gate_up_swiglu(gate, up, x), g / (1 + torch.exp(-g)) * u)
