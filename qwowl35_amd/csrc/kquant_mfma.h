@@ -916,6 +916,51 @@ struct KqPlan {
     int s = 1;  // K splits across workgroups (needs a workspace)
 };
 
+// Batch 3..8: row tiles per workgroup.  A launch runs in rounds of 256
+// workgroups, one per CU; a round takes the staging of the activation batch,
+// `stage` quarters of a tile's decode, and its tiles, so the tile count with the
+// fewest of rounds x (stage + 4 tiles) wins.  A plan of as many tiles as leave
+// one workgroup per CU, four above 768 row tiles, loses where that leaves a
+// round nearly empty: 17408 rows (1088 tiles) are two rounds of four, of which
+// the second is 16 workgroups, and five of one (us: 17408x2048 Q5_K b3 11.5 /
+// 13.5, 17408x8192 Q6_K b3 38.5 / 51.2; fused 17408x4096 GF2 b8 27.3 with three
+// tiles, 34.6 with two).  One sweep on one box of 1..4 tiles over 23 row counts, 15 k and every
+// codec at batch 3 and 8, plain and fused: this rule is within 1% of the fastest
+// on the mean, the fixed tile counts 3..20% by codec and form (fused q8_0 more
+// than twice).  stage: less where a tile takes longer (q8_0, the k-quants; two
+// matrices), more at batch 5..8.
+inline int batch_row_tiles(int fmt, int tiles, int chunks, int nb, bool swiglu) {
+    const bool light = fmt == kFmtGF4 || fmt == kFmtGF2, q8 = fmt == kFmtQ8, eight = nb >= 8;
+    int stage, most;
+    if (swiglu) {
+        // three fused q8_0 tiles spill in rounds
+        most = q8 && chunks > 16 ? 2 : 3;
+        stage = !q8                           ? (eight ? 1 + light : chunks > 8)
+                : chunks > 16 && chunks <= 24 ? (eight ? 3 : 1)
+                                              : 0;
+    } else {
+        // q8_0's tiles above these are slower by themselves (12288x5120 b3, us
+        // a round: one tile 6.9, two 11.3, three 23.4; 151936x2048 b8 three
+        // tiles 73.5 us, four 100)
+        most = !q8 ? 4 : eight ? (chunks <= 8 ? 3 : 4) : chunks > 8 && chunks <= 16 ? 3 : 2;
+        stage = !q8 ? (eight || light ? 2 : 1) : chunks > 8 ? 1 : eight ? 2 : 0;
+    }
+    int best = 1;
+    int64_t least = 0;
+    for (int rt = 1; rt <= most; ++rt) {
+        const int64_t groups = (tiles + rt - 1) / rt;
+        // beyond 16 rounds of one tile the CUs are no longer in step and a
+        // last round costs its share (head 100000x5120 GF4 b8, us: four tiles,
+        // 6.1 rounds, 88; three, 8.1 rounds, 96)
+        const int64_t cost = (tiles > 4096 ? groups : (groups + 255) / 256 * 256) * (stage + 4 * rt);
+        if (rt == 1 || cost < least) {
+            best = rt;
+            least = cost;
+        }
+    }
+    return best;
+}
+
 // KS waves x CPW chunks cover k with P chunks in flight per wave; RT row tiles
 // per workgroup amortise the per-chunk activation staging over more rows.
 // Settings from launch-shape sweeps on MI355X (graph replays, rotated weights),
@@ -944,20 +989,6 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
         if (split_ok && fmt != kFmtQ8 && tiles > 256 && tiles <= 384 && chunks > 48 && chunks % 2 == 0)
             return {3, 12, 2, 1, 2};
         if (chunks <= 4) return {1, 4, 1, 1};
-        if (chunks <= 8) {
-            // All of a row's chunks at once, one per wave: a second chunk per
-            // wave is never live, but the workgroup still loads it (chunk 0
-            // again) and waits for it (us, one chunk per wave against two:
-            // fused Q4_K 16384x2048 b8 14.3 / 19.8, b3 13.0 / 16.9; q8_0
-            // 151936x2048 b8 100 / 117, 7168x2048 b3 7.2 / 7.6).
-            if (tiles <= 256) return {1, 8, 1, 1};
-            if (tiles <= 512) return {2, 8, 1, 1};
-            if (tiles <= 768) return swiglu && fmt == kFmtQ8 && nb < 8 ? KqPlan{1, 8, 1, 1} : KqPlan{3, 8, 1, 1};
-            if (swiglu) return {2, 8, 1, 1};
-            // q8_0 at batch 3..4: one tile (greedy head 151936x2048 b3 80.7 us,
-            // with four tiles 111.4 in two chunks per wave; 32000x2048 22.2 / 28.6)
-            return fmt == kFmtQ8 && nb < 8 ? KqPlan{1, 8, 1, 1} : KqPlan{4, 8, 1, 1};
-        }
         if (kq_head_sized(rows, k) && !swiglu) {
             // at batch 8 four tiles per 4-wave workgroup (head b8
             // Q4_K 199 us, Q6_K 278, Q5_K 249, GF2 176; with {2, 4, 4, 2} 234 /
@@ -965,48 +996,54 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
             // us against 173.5 with four, 175.9 with six; Q6_K 258.7 with eight,
             // 240.3 with four)
             if (fmt == kFmtQ8) return {4, 8, 2, 1};
-            if (fmt == kFmtGF4) return {3, 8, 2, 1};
+            // GF4 at batch 3..4 with both chunks in flight (248320x4096 b3 116.9
+            // us against 122.3; at batch 8 217 against 150)
+            if (fmt == kFmtGF4) return nb >= 8 ? KqPlan{3, 8, 2, 1} : KqPlan{3, 8, 2, 2};
             if (nb >= 8 && fmt == kFmtQ4K) return {8, 4, 4, 1};
             return nb >= 8 ? KqPlan{4, 4, 4, 1} : KqPlan{2, 4, 4, 2};
         }
-        // Otherwise as many row tiles per workgroup as leave one workgroup per
-        // CU: the launch's time is a fixed start and tail, plus per round of
-        // workgroups the staging of the batch and the tiles.  One sweep on one
-        // box over 2048..13824 rows, k = 2560..17408 and every codec (b8, us,
-        // the plan here against the next best tile count): 6144x4096 (two
-        // tiles) q8_0 10.9 / 13.2, Q4_K 9.6 / 12.3; 10240x7168 (three) q8_0
-        // 23.7 / 29.3, Q5_K 21.0 / 27.3; 4096x5120 (one) GF4 8.9 / 9.9;
-        // fused 9728x2560 (three) GF4 12.1 / 15.0; one tile at any row count
-        // took 1.3-2 times as long where it needs several rounds.
-        // One or two tiles run one chunk per wave up to 16 chunks (4096x4096 b8
-        // q8_0 9.2 -> 8.6 us, 8192x4096 11.9 -> 11.5), longer rows on twelve
-        // waves in rounds; more tiles hold eight waves' loads.
-        if (tiles <= 256)
-            return chunks > 12 && chunks <= 16 ? KqPlan{1, 16, 1, 1} : KqPlan{1, 12, 2, 1};
-        // Fused q8_0, Q4_K and Q5_K of more than 24 chunks: two tiles in rounds
-        // need more registers than twelve waves leave (168 per lane; 96..104 of
-        // q8_0's spilled, 12..18 of the others'), so eight waves (us at b8,
-        // twelve / eight: 6144x8192 q8_0 85.8 / 33.6, Q4_K 30.2 / 25.1, Q5_K
-        // 34.2 / 28.2; GF4 and GF2 fit twelve).  q8_0 of more than two tiles
-        // per CU: one (12288x7168 b3 two on twelve waves 150, two on eight 52.6,
-        // one 42.9).
-        if (swiglu && chunks > 24 && tiles > 256 && fmt != kFmtGF4 && fmt != kFmtGF2 &&
-            (tiles <= 512 || tiles > 768 || fmt == kFmtQ8))
-            return fmt == kFmtQ8 && tiles > 512 ? KqPlan{1, 8, 2, 1} : KqPlan{2, 8, 2, 1};
-        if (tiles <= 512) {
-            // (two fused tiles per wave spill at sixteen waves)
-            return chunks > 12 && chunks <= 16 && !swiglu ? KqPlan{2, 16, 1, 1} : KqPlan{2, 12, 2, 1};
+        const int rt = batch_row_tiles(fmt, tiles, chunks, nb, swiglu);
+        const bool heavy = swiglu && fmt != kFmtGF4 && fmt != kFmtGF2;
+        // All of a row's chunks at once, one per wave: a second chunk per wave
+        // would never be live, but be loaded (chunk 0 again) and waited for
+        // (us, one chunk per wave against two: fused Q4_K 16384x2048 b8 14.3 /
+        // 19.8, q8_0 151936x2048 b8 100 / 117).
+        if (chunks <= 8) return {rt, 8, 1, 1};
+        // One round of at most two tiles: more waves, as the registers allow
+        // (us, against eight waves: {1, 16, 1, 1} 4096x4096 b8 Q4_K 8.4 / 9.2,
+        // {2, 16, 1, 1} 8192x4096 b8 Q5_K 11.0 / 12.1; two fused tiles spill at
+        // sixteen).  GF4 of 25..32 (batch 8: 28) chunks: one round of eight
+        // waves instead of two of twelve (4096x7168 b3 8.0 / 8.8).
+        if (tiles <= 256 * rt && rt == 1) {
+            if (chunks <= 16) return chunks <= 12 && swiglu ? KqPlan{1, 8, 2, 1} : KqPlan{1, 16, 1, 1};
+            if (fmt == kFmtGF4 && chunks > 24 && chunks <= (nb >= 8 ? 28 : 32)) return {1, 8, 4, 2};
+            return {1, 12, 2, 1};
         }
-        if (tiles <= 768) {
-            // fused q8_0: its five loads per tile and matrix spill in rounds,
-            // and at batch 3..4 one tile per workgroup is faster (12288x4096
-            // 24.6 us against 28.4; at batch 8 34.1 against 29.1)
-            if (swiglu && fmt == kFmtQ8 && chunks > 16) return {2, 12, 2, 1};
-            if (swiglu && fmt == kFmtQ8 && nb < 8) return {1, 8, 2, 1};
-            return {3, 8, 2, 1};
+        // 17..24 chunks on twelve waves are one pass over the row (8192x6144 b8
+        // q8_0 two tiles 17.3 us, on eight waves 19.2); with one tile per
+        // workgroup and several rounds, only fused q8_0 and, at batch 3..4, GF4
+        // gain by it.
+        if (chunks > 16 && chunks <= 24 &&
+            (rt == 2 || (rt == 1 && swiglu && (fmt == kFmtQ8 || (fmt == kFmtGF4 && nb < 8)))))
+            return {rt, 12, 2, 1};
+        // Longer rows in rounds.  Two fused tiles of q8_0, Q4_K and Q5_K need
+        // more registers then than twelve waves leave (168 per lane; 96..104 of
+        // q8_0's spilled, 12..18 of the others'; 6144x8192 b8, us, twelve / eight
+        // waves: q8_0 85.8 / 33.6, Q4_K 30.2 / 25.1, Q5_K 34.2 / 28.2).  Plain
+        // q8_0 takes twelve where they make few enough passes over the row
+        // (5120 rows b8: 48 chunks, two passes against three, 26.4 / 27.7; 28
+        // chunks, two against two, 20.0 / 18.0).
+        if (rt == 2 && chunks > 12) {
+            const bool one_round = tiles <= 512;
+            if (chunks <= 16) {
+                if (one_round && !swiglu) return {2, 16, 1, 1};
+                // (fused Q4_K and Q5_K also in several rounds, 2% faster)
+                if (swiglu && fmt != kFmtQ8 && (one_round || heavy)) return {2, 12, 2, 1};
+            } else if (one_round && !heavy) {
+                if (fmt != kFmtQ8 || 3 * ((chunks + 23) / 24) <= 2 * ((chunks + 15) / 16)) return {2, 12, 2, 1};
+            }
         }
-        if (swiglu) return {2, 12, 2, 1};
-        return {4, 8, 2, 1};
+        return {rt, 8, 2, 1};
     }
     // Longer rows: eight waves of four chunks per round (kq_mfma_gemv_long).
     if (chunks > 48) return {1, 8, 4, 2};
@@ -1143,32 +1180,40 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
                        ? kq_launch_cfg<FMT, NB, RT, KS, CPW, P, SWIGLU, true>(a, stream, p.s)      \
                        : kq_launch_cfg<FMT, NB, RT, KS, CPW, P, SWIGLU>(a, stream, p.s);           \
     }
+        constexpr bool kQ8 = FMT == kFmtQ8, kGF4 = FMT == kFmtGF4;
+        constexpr bool kHeavy = SWIGLU && !kGF4 && FMT != kFmtGF2;
         QW35_KQ_PLAN(1, 4, 1, 1)
         QW35_KQ_PLAN(1, 8, 1, 1)
-        QW35_KQ_PLAN(1, 16, 1, 1)
-        QW35_KQ_ROUNDS(1, 12, 2, 1)
         QW35_KQ_PLAN(2, 8, 1, 1)
-        QW35_KQ_PLAN(3, 8, 1, 1)
-        if constexpr (SWIGLU && FMT != kFmtGF4 && FMT != kFmtGF2) {
+        QW35_KQ_PLAN(1, 16, 1, 1)
+        QW35_KQ_ROUNDS(1, 8, 2, 1)
+        QW35_KQ_ROUNDS(1, 12, 2, 1)
+        QW35_KQ_ROUNDS(2, 8, 2, 1)
+        if constexpr (kHeavy) {
             QW35_KQ_PLAN(2, 12, 2, 1)
-            QW35_KQ_ROUNDS(2, 8, 2, 1)
         } else {
             QW35_KQ_ROUNDS(2, 12, 2, 1)
         }
-        if constexpr (SWIGLU && FMT == kFmtQ8) {
+        if constexpr (kGF4) { QW35_KQ_PLAN(1, 8, 4, 2) }
+        if constexpr (!kQ8 || SWIGLU || NB == 8) { QW35_KQ_PLAN(3, 8, 1, 1) }
+        if constexpr (kQ8 && (SWIGLU || NB == 4)) {
             QW35_KQ_PLAN(3, 8, 2, 1)
-            QW35_KQ_ROUNDS(1, 8, 2, 1)
         } else {
             QW35_KQ_ROUNDS(3, 8, 2, 1)
         }
         if constexpr (!SWIGLU) {
             QW35_KQ_PLAN(2, 16, 1, 1)
-            QW35_KQ_PLAN(4, 8, 1, 1)
-            QW35_KQ_ROUNDS(4, 8, 2, 1)
-            QW35_KQ_PLAN(4, 12, 1, 1)    // the K-split plans
-            if constexpr (FMT != kFmtQ8) { QW35_KQ_ROUNDS(3, 12, 2, 1) }
+            if constexpr (!kQ8) { QW35_KQ_PLAN(4, 8, 1, 1) }
+            if constexpr (kQ8 && NB == 4) {
+                QW35_KQ_PLAN(4, 8, 2, 1)
+            } else {
+                QW35_KQ_ROUNDS(4, 8, 2, 1)
+            }
+            QW35_KQ_PLAN(4, 12, 1, 1)  // the K-split plans
+            if constexpr (!kQ8) { QW35_KQ_ROUNDS(3, 12, 2, 1) }
+            if constexpr (kGF4 && NB == 4) { QW35_KQ_PLAN(3, 8, 2, 2) }
             if constexpr (FMT == kFmtQ4K && NB == 8) { QW35_KQ_PLAN(8, 4, 4, 1) }
-            if constexpr (FMT != kFmtQ8 && FMT != kFmtGF4) {
+            if constexpr (!kQ8 && !kGF4) {
                 if constexpr (NB == 8) {
                     QW35_KQ_PLAN(4, 4, 4, 1)
                 } else {

@@ -12,9 +12,12 @@ pytestmark = pytest.mark.gpu
 
 TYPES = {"gf4": 100, "gf2": 101, "q8_0": 8, "q4_k": 12, "q5_k": 13, "q6_k": 14}
 # rows, k, the plan's (row tiles, waves) for a plain GEMV at batch 3..8
-SHAPES = [(4096, 1536, (1, 8)), (4096, 2560, (1, 12)), (4088, 3584, (1, 16)), (1000, 5120, (1, 12)),
-          (4104, 1536, (2, 8)), (4104, 2560, (2, 12)), (8192, 3584, (2, 16)), (4104, 5120, (2, 12)),
+SHAPES = [(4096, 1536, (1, 8)), (4096, 2560, (1, 16)), (4088, 3584, (1, 16)), (1000, 5120, (1, 12)),
+          (4104, 1536, (2, 8)), (4104, 2560, (2, 8)), (8192, 3584, (2, 16)), (4104, 5120, (2, 12)),
           (8200, 2560, (3, 8)), (12288, 5120, (3, 8)), (12296, 1536, (4, 8)), (12296, 5120, (4, 8))]
+# q8_0, whose tiles take longer, where its plan differs
+Q8_PLANS = {(4104, 1536, 3): (1, 8), (12296, 1536, 3): (1, 8), (12296, 1536, 8): (2, 8), (12288, 5120, 3): (1, 8),
+            (12296, 5120, 3): (2, 12)}
 
 
 def _weight(name, rows, k, seed):
@@ -43,8 +46,8 @@ def test_batch_plans(cuda, name, rows, k, plan, nb):
     w = _weight(name, rows, k, rows + nb)
     kernel, args = rt.gemv_kernel(w, nb)["name"].split("<")
     if kernel != "gf4_mfma_gemv":  # (GF4 whose staged batch fits LDS runs its own kernel)
-        if name == "q8_0" and nb == 3 and k <= 2048 and plan[0] == 4:
-            plan = (1, 8)
+        if name == "q8_0":
+            plan = Q8_PLANS.get((rows, k, nb), plan)
         assert tuple(int(v) for v in args.split(",")[2:4]) == plan, args
     x = torch.randn((nb, k), device=cuda)
     awq = torch.rand(k, device=cuda) + 0.5
@@ -143,3 +146,22 @@ def test_fused_rounds(cuda, name, rows, k, nb):
     x = torch.randn((nb, k), device=cuda)
     g, u = (x.double() @ rt.dequantize(w).double().t() for w in (gate, up))
     _close(rt.ffn_gate_up_swiglu(gate, up, x), g / (1 + torch.exp(-g)) * u)
+
+
+@pytest.mark.parametrize("nb", [3, 8])
+@pytest.mark.parametrize("name,rows,k,plan", [
+    ("gf4", 1000, 7168, (1, 8, 4)),                                      # 28 chunks in one round of eight waves
+    ("gf4", 16392, 6400, (3, 8, 2)), ("q8_0", 4104, 6400, (2, 8, 2)),    # 1025 and 257 row tiles, 25 chunks
+    ("q4_k", 16392, 2560, None), ("q6_k", 16408, 6656, None), ("gf2", 16392, 5120, None)])
+def test_row_tile_rounds(cuda, name, rows, k, plan, nb):
+    """Row counts one past a round of workgroups, rows of one and of several passes."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    w = _weight(name, rows, k, rows + nb)
+    kernel, args = rt.gemv_kernel(w, nb)["name"].split("<")
+    if plan and kernel != "gf4_mfma_gemv":
+        assert tuple(int(v) for v in args.split(",")[2:5]) == plan, args
+    x = torch.randn((nb, k), device=cuda)
+    _close(rt.decode_matvec(w, x), x.double() @ rt.dequantize(w).double().t())

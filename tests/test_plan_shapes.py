@@ -61,14 +61,36 @@ def test_head_workspace_serves_smaller_batches(lib, type_id, rows, k):
 
 @pytest.mark.parametrize("type_id", [GF4, GF2, Q8, Q4K, Q5K, Q6K])
 @pytest.mark.parametrize("swiglu", [False, True])
-def test_short_rows_load_no_dead_chunk(lib, type_id, swiglu):
-    """Batch 3..8, rows of up to 2048 columns: no wave loads a chunk past the row."""
+def test_no_dead_chunk(lib, type_id, swiglu):
+    """Batch 3..8, rows of up to 4096 columns: no chunk that every wave loads lies past the row."""
     if swiglu and type_id == Q6K:
         pytest.skip("no fused q6_k")
     for rows in ROWS:
-        for chunks in (2, 4, 6, 8):
+        if rows >= 65536:  # (vocabulary-sized heads of 9..12 chunks have plans for 16)
+            continue
+        for chunks in (2, 4, 6, 8, 10, 12, 14, 16):
             for nb in range(3, 9):
                 name = kernel(type_id, rows, 256 * chunks, nb, swiglu=swiglu)
                 if name.startswith("kq_"):  # <codec, batch, row tiles, waves, chunks per wave, ...>
                     waves, per_wave = (int(v) for v in name.split("<")[1].split(",")[3:5])
                     assert (per_wave - 1) * waves < chunks, (rows, chunks, nb, name)
+
+
+@pytest.mark.parametrize("type_id", [GF4, GF2, Q8, Q4K, Q5K, Q6K])
+@pytest.mark.parametrize("swiglu", [False, True])
+def test_no_nearly_empty_round(lib, type_id, swiglu):
+    """Batch 3..8: the rounds of 256 workgroups that the row tiles of a launch
+    make run at most a third more tiles one after the other than the best count
+    of tiles per workgroup would (1088 row tiles: two rounds of four are eight,
+    five of one are five)."""
+    if swiglu and type_id == Q6K:
+        pytest.skip("no fused q6_k")
+    for rows in [r for r in ROWS if r < 65536] + [9728, 13824, 24576, 32000]:
+        tiles = -(-rows // 16)
+        serial = {rt: rt * -(-tiles // (256 * rt)) for rt in range(1, 5)}
+        for chunks in (6, 12, 16, 20, 32, 68):
+            for nb in range(3, 9):
+                name = kernel(type_id, rows, 256 * chunks, nb, swiglu=swiglu)
+                if name.startswith("kq_"):
+                    rt = int(name.split("<")[1].split(",")[2])
+                    assert serial[rt] <= 4 / 3 * min(serial.values()), (rows, chunks, nb, name)
