@@ -933,17 +933,18 @@ inline int batch_row_tiles(int fmt, int tiles, int chunks, int nb, bool swiglu) 
     const bool light = fmt == kFmtGF4 || fmt == kFmtGF2, q8 = fmt == kFmtQ8, eight = nb >= 8;
     int stage, most;
     if (swiglu) {
-        // three fused q8_0 tiles spill in rounds
-        most = q8 && chunks > 16 ? 2 : 3;
-        stage = !q8                           ? (eight ? 1 + light : chunks > 8)
-                : chunks > 16 && chunks <= 24 ? (eight ? 3 : 1)
-                                              : 0;
+        // fused q8_0, and at batch 3..4 rows of up to eight chunks: one tile, as
+        // staging weighs nothing against two matrices' tiles (three fused q8_0
+        // tiles also spill in rounds); 17..24 chunks on twelve waves are one pass
+        // over the row with two
+        most = q8 ? (chunks > 16 && chunks <= 24 ? 2 : 1) : eight || chunks > 8 ? 3 : 1;
+        stage = q8 ? (eight ? 3 : 1) : eight ? 1 + light : 1;
     } else {
         // q8_0's tiles above these are slower by themselves (12288x5120 b3, us
         // a round: one tile 6.9, two 11.3, three 23.4; 151936x2048 b8 three
         // tiles 73.5 us, four 100)
-        most = !q8 ? 4 : eight ? (chunks <= 8 ? 3 : 4) : chunks > 8 && chunks <= 16 ? 3 : 2;
-        stage = !q8 ? (eight || light ? 2 : 1) : chunks > 8 ? 1 : eight ? 2 : 0;
+        most = !q8 ? 4 : eight ? (chunks <= 8 ? 3 : 4) : chunks <= 8 ? 1 : chunks <= 16 ? 3 : 2;
+        stage = !q8 ? (eight || light ? 2 : 1) : eight && chunks <= 8 ? 2 : 1;
     }
     int best = 1;
     int64_t least = 0;
@@ -1180,44 +1181,55 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
                        ? kq_launch_cfg<FMT, NB, RT, KS, CPW, P, SWIGLU, true>(a, stream, p.s)      \
                        : kq_launch_cfg<FMT, NB, RT, KS, CPW, P, SWIGLU>(a, stream, p.s);           \
     }
-        constexpr bool kQ8 = FMT == kFmtQ8, kGF4 = FMT == kFmtGF4;
-        constexpr bool kHeavy = SWIGLU && !kGF4 && FMT != kFmtGF2;
-        QW35_KQ_PLAN(1, 4, 1, 1)
-        QW35_KQ_PLAN(1, 8, 1, 1)
-        QW35_KQ_PLAN(2, 8, 1, 1)
+        // what batch_row_tiles and plan_kq take for the codec, batch and form (a
+        // plain GF4 plan of up to 16 chunks is the greedy head's only)
+        constexpr bool kQ8 = FMT == kFmtQ8, kGF4 = FMT == kFmtGF4, kLight = kGF4 || FMT == kFmtGF2;
+        constexpr bool kHeavy = SWIGLU && !kLight, kEight = NB == 8;
+        if constexpr (!SWIGLU || !kGF4) {
+            QW35_KQ_PLAN(1, 4, 1, 1)
+            QW35_KQ_PLAN(1, 8, 1, 1)
+        }
+        if constexpr (kQ8 ? kEight && !SWIGLU : !SWIGLU || (kEight && !kGF4)) {
+            QW35_KQ_PLAN(2, 8, 1, 1)
+            QW35_KQ_PLAN(3, 8, 1, 1)
+        }
         QW35_KQ_PLAN(1, 16, 1, 1)
-        QW35_KQ_ROUNDS(1, 8, 2, 1)
+        if constexpr (kQ8 || (!kLight && (SWIGLU || !kEight)) || (kLight && SWIGLU && !kEight)) {
+            QW35_KQ_ROUNDS(1, 8, 2, 1)
+        } else if constexpr (SWIGLU) {
+            QW35_KQ_PLAN(1, 8, 2, 1)
+        }
         QW35_KQ_ROUNDS(1, 12, 2, 1)
-        QW35_KQ_ROUNDS(2, 8, 2, 1)
         if constexpr (kHeavy) {
             QW35_KQ_PLAN(2, 12, 2, 1)
         } else {
             QW35_KQ_ROUNDS(2, 12, 2, 1)
         }
         if constexpr (kGF4) { QW35_KQ_PLAN(1, 8, 4, 2) }
-        if constexpr (!kQ8 || SWIGLU || NB == 8) { QW35_KQ_PLAN(3, 8, 1, 1) }
-        if constexpr (kQ8 && (SWIGLU || NB == 4)) {
+        if constexpr (!kQ8 || !SWIGLU) { QW35_KQ_ROUNDS(2, 8, 2, 1) }
+        if constexpr (kQ8 && !SWIGLU && !kEight) {
             QW35_KQ_PLAN(3, 8, 2, 1)
-        } else {
+            QW35_KQ_PLAN(4, 8, 2, 1)
+        } else if constexpr (!kQ8 || !SWIGLU) {
             QW35_KQ_ROUNDS(3, 8, 2, 1)
+            if constexpr (!SWIGLU) { QW35_KQ_ROUNDS(4, 8, 2, 1) }
         }
         if constexpr (!SWIGLU) {
             QW35_KQ_PLAN(2, 16, 1, 1)
             if constexpr (!kQ8) { QW35_KQ_PLAN(4, 8, 1, 1) }
-            if constexpr (kQ8 && NB == 4) {
-                QW35_KQ_PLAN(4, 8, 2, 1)
-            } else {
-                QW35_KQ_ROUNDS(4, 8, 2, 1)
+            QW35_KQ_PLAN(4, 12, 1, 1)  // the K-split plans; the second is of 25 chunks or more a split
+            if constexpr (!kQ8) {
+                if (p.rt == 3 && p.ks == 12)
+                    return kq_launch_cfg<FMT, NB, 3, 12, 2, 1, SWIGLU, true>(a, stream, p.s);
             }
-            QW35_KQ_PLAN(4, 12, 1, 1)  // the K-split plans
-            if constexpr (!kQ8) { QW35_KQ_ROUNDS(3, 12, 2, 1) }
-            if constexpr (kGF4 && NB == 4) { QW35_KQ_PLAN(3, 8, 2, 2) }
-            if constexpr (FMT == kFmtQ4K && NB == 8) { QW35_KQ_PLAN(8, 4, 4, 1) }
+            // the vocabulary-sized heads
+            if constexpr (kGF4 && !kEight) { QW35_KQ_PLAN(3, 8, 2, 2) }
+            if constexpr (FMT == kFmtQ4K && kEight) { QW35_KQ_PLAN(8, 4, 4, 1) }
             if constexpr (!kQ8 && !kGF4) {
-                if constexpr (NB == 8) {
-                    QW35_KQ_PLAN(4, 4, 4, 1)
-                } else {
+                if constexpr (!kEight) {
                     QW35_KQ_PLAN(2, 4, 4, 2)
+                } else if constexpr (FMT != kFmtQ4K) {
+                    QW35_KQ_PLAN(4, 4, 4, 1)
                 }
             }
         }
@@ -1225,11 +1237,14 @@ hipError_t kq_launch_nb(const GemvArgs& a, hipStream_t stream) {
     } else {
         if ((a.k >> 8) > 48)  // the long-row plan, in rounds of 32 chunks
             return kq_launch_cfg<FMT, NB, 1, 8, 4, (kq_fits<FMT, NB, 1, 2, SWIGLU>() ? 2 : 1), SWIGLU, true>(a, stream);
-        QW35_KQ_PLAN(1, 4, 1, 1)
-        QW35_KQ_PLAN(1, 8, 1, 1)
-        QW35_KQ_PLAN(1, 8, 2, 2)
-        QW35_KQ_PLAN(1, 8, 4, 2)
-        QW35_KQ_PLAN(1, 8, 6, 2)
+        // (fused GF4 of up to 48 chunks runs its own kernel)
+        if constexpr (FMT != kFmtGF4 || !SWIGLU) {
+            QW35_KQ_PLAN(1, 4, 1, 1)
+            QW35_KQ_PLAN(1, 8, 1, 1)
+            QW35_KQ_PLAN(1, 8, 2, 2)
+            QW35_KQ_PLAN(1, 8, 4, 2)
+            if constexpr (FMT == kFmtQ8 || FMT == kFmtGF4) { QW35_KQ_PLAN(1, 8, 6, 2) }
+        }
         if constexpr (FMT == kFmtQ8) { QW35_KQ_PLAN(1, 16, 1, 1) }
         // Fused gate/up holds two matrices' loads per tile: more than two row
         // tiles per workgroup spill registers, so those take the one-tile

@@ -165,3 +165,21 @@ def test_row_tile_rounds(cuda, name, rows, k, plan, nb):
         assert tuple(int(v) for v in args.split(",")[2:5]) == plan, args
     x = torch.randn((nb, k), device=cuda)
     _close(rt.decode_matvec(w, x), x.double() @ rt.dequantize(w).double().t())
+
+
+@pytest.mark.parametrize("nb", [1, 2, 3, 8])
+@pytest.mark.parametrize("rows", [1000, 4104, 8200, 12304, 16392, 65552])
+def test_gf4_head_plans(cuda, rows, nb):
+    """The GF4 greedy head runs the chunked kernel at every batch and length, the GF4 GEMV its own."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    for k in (1024, 1536, 2560, 3584, 6400) if rows < 65536 else (2560,):
+        w = _weight("gf4", rows, k, k)
+        x = torch.randn((nb, k), device=cuda)
+        want = x.double() @ rt.dequantize(w).double().t()
+        token, logit = rt.output_argmax(w, x)
+        best = want.max(dim=1)
+        assert torch.equal(token.long(), best.indices), k
+        assert float((logit.double() - best.values).abs().max()) <= 2e-6 * float(want.norm(dim=1).max())

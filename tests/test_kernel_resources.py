@@ -7,11 +7,13 @@ q8_0 12288x7168 at batch 8: 151 us with 99 spilled registers, 58 without).
 The built library carries each kernel's counts in its code objects' notes."""
 from __future__ import annotations
 
+import re
 import struct
 
 import msgpack
 
 from qwowl35_amd import build
+from tests.test_plan_coverage import GF2, Q4K, Q5K, Q6K, Q8, kernel
 
 
 def _kernels(blob: bytes):
@@ -45,3 +47,27 @@ def test_no_gemv_kernel_spills_registers():
     assert len(kernels) > 100
     spilled = {k[".name"]: k[".vgpr_spill_count"] for k in kernels if k[".vgpr_spill_count"]}
     assert not spilled, spilled
+
+
+def test_every_chunked_gemv_kernel_is_launched():
+    """No instantiation of the chunked kernel that no shape launches (GF4 left
+    out: its plain ones are the greedy head's, which is not described here)."""
+    built = set()
+    for k in _kernels(build.LIB.read_bytes()):
+        m = re.search(r"(kq_mfma_gemv(?:_long)?)I(\w+?)EEv", k[".name"])
+        if m:
+            args = [n or ("true" if b == "1" else "false") for n, b in re.findall(r"Li(\d+)E|Lb(\d)", m.group(2))]
+            if args[0] != "2" and args[-1] == "false":  # (the other half takes an AWQ multiplier)
+                built.add(f"{m.group(1)}<{', '.join(args)}>")
+    tiles = [1, 257, 385, 513, 640, 769, 832, 1025, 1089, 1281, 1344, 1537, 1664, 2049, 3073, 4096, 4097, 6250]
+    chunks = [2, 4, 6, 8, 10, 12, 14, 16, 18, 24, 26, 28, 32, 40, 48, 50, 52, 68]
+    launched = set()
+    for t in (GF2, Q8, Q4K, Q5K, Q6K):
+        for swiglu in (False, True):
+            for n in tiles if not (swiglu and t == Q6K) else []:
+                for c in chunks:
+                    for nb in (1, 2, 3, 8):
+                        launched.add(kernel(t, 16 * n, 256 * c, nb, swiglu=swiglu))
+                        if c >= 48:
+                            launched.add(kernel(t, 16 * n, 256 * c, nb, swiglu=swiglu, ws=True).split("+")[0])
+    assert built and built <= launched, sorted(built - launched)
