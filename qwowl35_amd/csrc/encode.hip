@@ -197,7 +197,7 @@ __global__ __launch_bounds__(kEncodeThreads) void gf2_pack_kernel(const float* _
             if (i0 + u >= n_blocks) break;
             float amax = fmaxf(fmaxf(fabsf(v[u][0]), fabsf(v[u][1])), fmaxf(fabsf(v[u][2]), fabsf(v[u][3])));
             amax = dpp_fmax<kDppQuadXor1>(amax);
-            amax = dpp_fmax<kDppQuadXor2>(amax);
+            amax = fmaxf(dpp_fmax<kDppQuadXor2>(amax), 0.0f);  // (a group of NaN: zero, also below)
             const uint32_t b = ((f32_to_f16_bits(amax) + 0x80u) >> 8) & 0xFFu;
             const float s = f16_bits_to_f32(b << 8);
             float r[4];
@@ -259,7 +259,7 @@ __global__ __launch_bounds__(kEncodeThreads) void q8_0_quantize_kernel(const flo
             amax = dpp_fmax<kDppRowHalfMirror>(dpp_fmax<kDppQuadXor2>(dpp_fmax<kDppQuadXor1>(amax)));
             amax_u = (lane & 3) == u ? amax : amax_u;
         }
-        const float d_u = __fdiv_rn(amax_u, 127.0f);
+        const float d_u = __fdiv_rn(fmaxf(amax_u, 0.0f), 127.0f);
         const float inv_u = (d_u != 0.0f) ? __fdiv_rn(1.0f, d_u) : 0.0f;
 #pragma unroll
         for (int u = 0; u < kSuperUnroll; ++u) {
@@ -322,6 +322,7 @@ __global__ __launch_bounds__(kEncodeThreads) void k_quantize_kernel(const float*
             hi_u = (lane & 3) == u ? hi : hi_u;
         }
         lo_u = fminf(lo_u, 0.0f);
+        hi_u = fmaxf(hi_u, -__builtin_inff());  // (a sub-block of NaN: the maximum of no elements)
         const float scale = __fdiv_rn(__fsub_rn(hi_u, lo_u), kLevels);
         const float mins = -lo_u;
         float smax = scale, mmax = mins;
@@ -422,6 +423,7 @@ __global__ __launch_bounds__(kEncodeThreads) void q6_k_quantize_kernel(const flo
             amax = dpp_fmax<kDppQuadXor2>(dpp_fmax<kDppQuadXor1>(amax));
             amax_u = (lane & 3) == u ? amax : amax_u;
         }
+        amax_u = fmaxf(amax_u, 0.0f);
         const float sub = __fdiv_rn(amax_u, 31.0f);
         float smax = sub;
 #pragma unroll

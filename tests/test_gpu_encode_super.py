@@ -62,3 +62,35 @@ def test_sub_blocks_far_below_the_largest(cuda, name):
     got = rt.quantize(torch.from_numpy(v).to(cuda), CODECS[name]).cpu().numpy().reshape(rows, -1)
     want = oq6.q6_k_quantize(v) if name == "q6_k" else om.quantize(CODECS[name], v)
     assert np.array_equal(got, np.asarray(want).reshape(rows, -1).view(np.uint8))
+
+
+@pytest.mark.parametrize("name", [*CODECS, "q8_0"])
+def test_groups_of_nan(cuda, name):
+    """A scale group with no number in it (outside the contract, src must be
+    finite): its largest magnitude is that of no elements, zero, as the NaN of a
+    group beside numbers is passed over, so one such group neither spreads to
+    the super-block's scale nor becomes a NaN scale itself."""
+    import torch
+
+    from qwowl35_amd import runtime as rt
+
+    rng = np.random.default_rng(3)
+    w = rng.standard_normal((4, 512)).astype(np.float32)
+    w[0, 32:64] = np.nan    # whole groups of every codec (16 or 32 columns)
+    w[1, 7] = np.nan        # one element
+    w[2, :256] = np.nan     # a whole super-block
+    zeros = w.copy()
+    zeros[0, 32:64] = 0.0
+    zeros[2, :256] = 0.0
+    type_id = {**CODECS, "q8_0": om.TYPE_Q8_0}[name]
+    got, want = (rt.quantize(torch.from_numpy(v).to(cuda), type_id).cpu().numpy().reshape(4, -1).copy()
+                 for v in (w, zeros))
+    if name == "q8_0":  # a scale of zero, codes of -127 (NaN * 0, clamped) where zeros have 0
+        for v in (got, want):
+            blocks = v.reshape(4, 16, 34)
+            blocks[0, 1, 2:] = blocks[2, :8, 2:] = 0
+    if name in ("q4_k", "q5_k"):  # the range of no elements is -inf, its minimum -0
+        block = got[2, :got.shape[1] // 2]
+        assert block[:4].tobytes() == b"\x00\xfc\x00\x80" and not block[4:].any()
+        got[2], want[2] = 0, 0
+    assert np.array_equal(got, want)
