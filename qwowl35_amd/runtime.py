@@ -206,9 +206,20 @@ def _ptr(t: torch.Tensor | None) -> C.c_void_p:
     return C.c_void_p(t.data_ptr() if t is not None else None)
 
 
+def _raw_stream_of(binding):
+    """The current stream's handle by device index: without a torch.cuda.Stream
+    object for each call (a third of a small GEMV's host time) where ``binding``
+    (``torch._C``) has torch's private accessor, else through the public one."""
+    fast = getattr(binding, "_cuda_getCurrentRawStream", None)
+    return fast if fast is not None else lambda device: torch.cuda.current_stream(device).cuda_stream
+
+
+_raw_stream = _raw_stream_of(torch._C)
+
+
 def _stream(stream) -> C.c_void_p:
-    if stream is None:  # the current stream's handle, without a torch.cuda.Stream object for each call
-        return C.c_void_p(torch._C._cuda_getCurrentRawStream(torch.cuda.current_device()))
+    if stream is None:
+        return C.c_void_p(_raw_stream(torch.cuda.current_device()))
     return C.c_void_p(stream.cuda_stream)
 
 
