@@ -1,6 +1,6 @@
 """The batch 3..8 GEMV plans at the edges where the row-tile count per workgroup
-or the wave count changes: 256 / 512 / 768 row tiles of 16, 8 / 12 / 16 / 24 and
-48 chunks of 256 columns, and the K split of longer rows.  Each output against
+or the wave count changes: 256 / 512 / 768 / 1024 row tiles of 16, 8 / 12 / 16 /
+24 chunks of 256 columns, and the K split of longer rows.  Each output against
 an fp64 product of the library's dequantised weights (bit-exact against the
 oracle in the other tests) within 1e-6 relative L2 plus, for GF2's thirds and
 the fp16 hi/lo activations, their 2^-22: 2e-6."""
@@ -82,7 +82,10 @@ def test_long_rows_split(cuda, name, rows):
 
     k, nb = 13312, 5
     w = _weight(name, rows, k, rows)
-    assert rt.gemv_kernel(w, nb, workspace=True)["workspace_bytes"] > 0
+    plan = rt.gemv_kernel(w, nb, workspace=True)
+    assert plan["workspace_bytes"] > 0
+    assert plan["name"].startswith("kq_mfma_gemv_long<") and plan["name"].split(",")[2:4] == [" 3", " 12"], plan
+    assert plan["grid"] == 2 * -(-rows // 48)  # two workgroups per group of three row tiles
     ws = rt.decode_matvec_workspace(w, nb, device=cuda)
     x = torch.randn((nb, k), device=cuda)
     y = rt.decode_matvec(w, x, workspace=ws)

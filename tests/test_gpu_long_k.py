@@ -5,12 +5,13 @@ The reference's decode takes any k through n_blocks = ceil(k / block)
 (qw35-server/src/metal/bridge/Qw35MetalRuntime+FFN.m:240), and its tiled
 prefill matmul loops over K.  Here a decode GEMV whose row is longer than its
 plan covers in one round runs as kq_mfma_gemv_long (rounds of 8 waves x 4
-chunks), and the prefill staging pass reads rows past 12288 columns twice.
+chunks at batch 1..2, of 12 waves x 2 for the row counts here at batch 3..8),
+and the prefill staging pass reads rows past 24576 columns twice.
 Bars are those of the 9B shapes: GEMVs within GEMV_REL_L2 of the fp64 matvec of
 the oracle-dequantised weights; prefill within 1e-3 relative L2 (fp32 output)
 or one bf16 ulp plus the fp32-accumulation allowance (bf16 output) of the
 fp64 product of the operands the kernel contracts.  k = 17408 = 68 chunks
-leaves the last round four chunks long (waves partly idle)."""
+leaves the last round four (batch 1..2) or twenty chunks long (waves partly idle)."""
 from __future__ import annotations
 
 import numpy as np
@@ -52,7 +53,7 @@ def test_long_k_gemv_parity(cuda, name, nb):
     x = activations(rng, nb, k)
     y = _rt().decode_matvec(w, _t(x, cuda)).cpu().numpy()
     assert om.rel_l2(y, om.matvec_f64(deq, x)) <= GEMV_REL_L2
-    # AWQ + residual, and the K-split entry point (no split plan at this k: same kernel)
+    # AWQ + residual, and the K-split entry point (no split plan at this row count: same kernel)
     a = awq_scales(rng, k)
     base = rng.standard_normal((nb, rows)).astype(np.float32)
     dst = torch.from_numpy(base.copy()).to(cuda)
