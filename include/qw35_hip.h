@@ -159,13 +159,14 @@ int qw35_hip_ffn_gate_up_swiglu(const qw35_hip_weight *gate, const qw35_hip_weig
                                 uintptr_t err_len);
 
 /* Decode GEMV with a K-split workspace (otherwise qw35_hip_decode_matvec):
- * at batch 3..8 on k = 12288 matrices of at most 4096 rows (the down
- * projection) every workgroup of the plain launch would convert the whole
- * activation batch, so with a workspace the launch splits K four ways across
- * workgroups of four row tiles; each writes its partial sums to the workspace
- * and the last of a
- * row group to finish adds them in a fixed order (so results do not depend
- * on timing) and writes dst.  workspace: device memory of at least
+ * at batch 3..8 every workgroup of the plain launch converts the whole
+ * activation batch.  With a workspace the launch splits K across workgroups of
+ * several row tiles where that is faster: four ways for k = 12288 matrices of
+ * at most 4096 rows (the 9B's down projection), two ways for matrices of
+ * 4097..6144 rows with k above 12288 and a multiple of 512 (not q8_0); each
+ * workgroup writes its partial sums to the workspace and the last of a row
+ * group to finish adds them in a fixed order (so results do not depend on
+ * timing) and writes dst.  workspace: device memory of at least
  * qw35_hip_decode_matvec_workspace_size(w, n_batch) bytes (0: this call never
  * splits; a smaller workspace disables the split), 256-byte aligned,
  * zero-filled before its first use; its first 1 KiB holds the row-group

@@ -902,7 +902,8 @@ __global__ __launch_bounds__(64 * KS) void kq_mfma_gemv(GemvArgs args) {
     kq_gemv_body<FMT, NB, RT, KS, CPW, P, SWIGLU, HAS_AWQ, false>(args);
 }
 
-// Rows longer than one round covers (k beyond 12288 columns).
+// Rows longer than one round of the plan's KS x CPW chunks covers: k beyond
+// 12288 columns at batch 1..2, beyond 4096 or 6144 at batch 3..8.
 template <int FMT, int NB, int RT, int KS, int CPW, int P, bool SWIGLU, bool HAS_AWQ>
 __global__ __launch_bounds__(64 * KS) void kq_mfma_gemv_long(GemvArgs args) {
     kq_gemv_body<FMT, NB, RT, KS, CPW, P, SWIGLU, HAS_AWQ, true>(args);
@@ -985,8 +986,8 @@ inline KqPlan plan_kq(int fmt, int rows, int k, int nb, bool split_ok = false, b
         if (split_ok && tiles <= 256 && chunks == 48) return {4, 12, 1, 1, 4};
         // Longer rows of 257..384 tiles: three tiles and two splits keep one
         // workgroup per CU (5120x17408 b8, us, against two unsplit tiles: GF4
-        // 22.6 / 25.1, Q4_K 24.9 / 27.3, Q5_K 27.5 / 30.5, GF2 22.8 / 26.9;
-        // q8_0 51 / 35.0).
+        // 22.6 / 25.1, Q4_K 24.9 / 27.3, Q5_K 27.5 / 30.5, GF2 22.8 / 26.9, Q6_K
+        // 29.8 / 33.2; q8_0 51 / 35.0).
         if (split_ok && fmt != kFmtQ8 && tiles > 256 && tiles <= 384 && chunks > 48 && chunks % 2 == 0)
             return {3, 12, 2, 1, 2};
         if (chunks <= 4) return {1, 4, 1, 1};
@@ -1079,7 +1080,9 @@ size_t kq_lds_bytes() {
 // K-split workspace: kKsCounters row-group counters at its start (the same
 // place for every shape, so a launch always finds the counters the previous
 // one returned to zero), then the partials (one RT x NB x 16 x NM block per
-// workgroup).  Split plans cover at most 256 row tiles, so at most 256 groups.
+// workgroup).  Split plans cover at most 256 row tiles in groups of four, or 384
+// in groups of three, and a few ragged groups more where segments share the
+// launch; a launch of more groups than counters takes the unsplit plan.
 constexpr int kKsCounters = 256;
 constexpr size_t kKsPartOffset = kKsCounters * 4;
 inline size_t kq_split_ws_bytes(int groups, int splits, int rt, int nb, int nm) {
