@@ -312,8 +312,12 @@ def _refuse_unchunked(w: HipWeight, what: str) -> None:
 
 
 def output_argmax_workspace(w: HipWeight, n_batch: int, device="cuda") -> torch.Tensor:
-    """Device bytes for ``output_argmax`` (size from the C ABI, +256 for alignment)."""
-    need = int(_ffi.load().qw35_hip_output_argmax_workspace_size(C.byref(w.view), n_batch))
+    """Device bytes for ``output_argmax`` of up to ``n_batch`` rows (the largest
+    of the C ABI's sizes over those batches, +256 for alignment)."""
+    size = _ffi.load().qw35_hip_output_argmax_workspace_size
+    need = int(size(C.byref(w.view), n_batch))
+    if need:  # (0: a batch the head refuses)
+        need = max(int(size(C.byref(w.view), b)) for b in range(1, n_batch + 1))
     if need == 0:
         _refuse_unchunked(w, "output_argmax")
         raise Qw35Error("output_argmax: invalid weight or batch")
@@ -332,8 +336,8 @@ def output_argmax(w: HipWeight, x: torch.Tensor, awq: torch.Tensor | None = None
     if need == 0:
         _refuse_unchunked(w, "output_argmax")
         raise Qw35Error("output_argmax: invalid weight or batch")
-    if workspace is None:
-        workspace = output_argmax_workspace(w, nb, device=x.device)
+    if workspace is None:  # this call's own
+        workspace = torch.empty(need + 256, dtype=torch.uint8, device=x.device)
     base = workspace.data_ptr()
     pad = (-base) % 256
     if workspace.numel() - pad < need:

@@ -94,3 +94,21 @@ def test_no_nearly_empty_round(lib, type_id, swiglu):
                 if name.startswith("kq_"):
                     rt = int(name.split("<")[1].split(",")[2])
                     assert serial[rt] <= 4 / 3 * min(serial.values()), (rows, chunks, nb, name)
+
+
+@pytest.mark.parametrize("type_id", [GF4, GF2, Q8, Q4K, Q5K, Q6K])
+@pytest.mark.parametrize("rows,k", [(65552, 4096), (248320, 4096), (151936, 2560), (32000, 2048)])
+def test_head_workspace_tensor_serves_smaller_batches(lib, type_id, rows, k):
+    """The runtime's workspace tensor also where the C ABI's size is that of one batch (vocabulary-sized heads)."""
+    from qwowl35_amd import runtime as rt
+
+    w = _ffi.Weight()
+    w.data, w.k, w.rows, w.type_id, w.bytes = 256, k, rows, type_id, ROW_BYTES[type_id](k) * rows
+    head = rt.HipWeight(None, w)
+    for n in range(1, 9):
+        numel = rt.output_argmax_workspace(head, n, device="cpu").numel()
+        for nb in range(1, n + 1):
+            assert numel - 256 >= lib.qw35_hip_output_argmax_workspace_size(C.byref(w), nb), (n, nb)
+    for bad in (0, 9):
+        with pytest.raises(_ffi.Qw35Error, match="invalid weight or batch"):
+            rt.output_argmax_workspace(head, bad, device="cpu")
